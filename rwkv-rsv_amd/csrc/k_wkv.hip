@@ -832,184 +832,33 @@ int launch_wkv7_seq_ragged(rsv_ctx *ctx, float *s, const float *r, const float *
 
 // ------------------------------------- ragged prefill scan, gated fp16 out
 // The scan of rsv_wkv7_seq_ragged_gate, leaving the att.output operand
-// yg = (GroupNorm(y) + bonus*v) * g in fp16: k_wkv7_seq_rows writes the raw
+// yg = (GroupNorm(y) + bonus*v) * g in fp16: a scan (k_wkv7_seq_mm 16 tokens at
+// a time, k_wkv7_seq_cols token by token for short segments) writes the raw
 // y = S r and the head's bonus sum per token, then k_gn_gate_f16 applies
-// GroupNorm + bonus*v and the gate.  Per (head, segment), 64/RPL lane groups
-// of four lanes: a group owns RPL state rows, each lane 16 columns of them.
-// The head's column vectors of a batch of tokens (the reductions over the
-// head, |k| and the bonus sum, included) are formed four tokens per wave
-// into LDS first, so the scan's dependent chain per token is the row-local
-// update alone.  Against the one-wave scan with GroupNorm inside
-// (k_wkv7_seq_ragged): 560 -> 333 us on 8 segments of 512 tokens (40
-// heads), 227 -> 211 us on 64 of 64.
-template <int RPL>
-__global__ __launch_bounds__(256 / RPL) void k_wkv7_seq_rows(
+// GroupNorm + bonus*v and the gate.
+//
+// Token by token: one state row per group of 8 lanes, each lane 8 columns,
+// 8 waves per (head, segment).  The head's column vectors of a batch of tokens
+// (the reductions over the head, |k| and the bonus sum, included) are formed
+// one token per wave into LDS first (8 per batch), so the dependent chain per
+// token is 8 multiply-adds and a 3-step DPP sum.  Its per-token latency bounds
+// it: 128 segments of one token 34 us, 40 heads (45 with four lanes and two
+// rows per group), 64 of 24 tokens 86 (89), 24 of 21 39 (42; 43 with 16 lanes).
+__device__ __forceinline__ float oct_sum(float v) {
+    v += quad_dpp<0xB1>(v);      // quad_perm 1,0,3,2
+    v += quad_dpp<0x4E>(v);      // quad_perm 2,3,0,1
+    return v + quad_dpp<0x141>(v);  // row_half_mirror: the 8-lane sum in every lane of the 8
+}
+
+__global__ __launch_bounds__(512) void k_wkv7_seq_cols(
     float *__restrict__ S, const float *__restrict__ r, const float *__restrict__ w, const float *__restrict__ k,
     const float *__restrict__ v, const float *__restrict__ a, const float *__restrict__ kkc,
     const float *__restrict__ ka, const float *__restrict__ rk, float *__restrict__ y_out,
     float *__restrict__ bonus_out, const uint32_t *__restrict__ seg_start, const uint32_t *__restrict__ seg_len,
     const uint32_t *__restrict__ seg_slot, int H, float eps, uint64_t rows, uint64_t slots) {
-    constexpr int NW = 4 / RPL;   // waves per (head, segment)
-    constexpr int kRB = 4 * NW;   // tokens per batch: four per wave in the batch phase
-    // per batch: [token][k^ | -k^ a | w | k_mod | r | v] x 64 columns, two batches alternating
-    __shared__ __attribute__((aligned(16))) float hb[2][kRB][6 * 64];
-    // the batch's outputs (y per token and row, the bonus sum per token) are
-    // staged in LDS and stored once the batch is done: a global store per
-    // token would hold its data register until the write completes
-    __shared__ __attribute__((aligned(16))) float yl[2][kRB][64];
-    __shared__ float bl[2][kRB];
-    const int h = blockIdx.x, gi = blockIdx.y, tid = threadIdx.x;
-    const int wave = tid >> 6, lane = tid & 63, q = lane & 3;
-    const int row0 = 16 * RPL * wave + RPL * (lane >> 2);  // this lane's rows row0 .. row0 + RPL - 1
-    const size_t C = (size_t)H * 64;
-    const uint32_t t0 = seg_start[gi], len = seg_len[gi], slot = seg_slot[gi];
-    if (slot >= slots || (uint64_t)t0 + len > rows) return;  // uniform per block
-    float4 *Sb = (float4 *)(S + ((size_t)slot * H + h) * 4096);
-    float s[RPL][16];
-#pragma unroll
-    for (int i = 0; i < RPL; i++)
-#pragma unroll
-        for (int m = 0; m < 4; m++) {
-            const float4 x = Sb[(row0 + i) * 16 + 4 * q + m];
-            s[i][4 * m] = x.x; s[i][4 * m + 1] = x.y; s[i][4 * m + 2] = x.z; s[i][4 * m + 3] = x.w;
-        }
-    // column role (batch phase): lane j forms column j's vectors of tokens
-    // 4*wave .. 4*wave+3 of a batch; every reduction over the head happens
-    // here, for four tokens at once, off the scan's dependent chain
-    const int j = lane;
-    const float kkc_j = kkc[h * 64 + j], ka_j = ka[h * 64 + j], rk_j = rk[h * 64 + j];
-    float pk[4], pa[4], pw[4], pr[4], pv[4];
-    auto load_batch = [&](uint32_t tb) {
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-            const uint32_t t = tb + 4 * wave + i;
-            const size_t vo = (size_t)(t0 + (t < len ? t : 0)) * C + (size_t)h * 64 + j;
-            pk[i] = k[vo]; pa[i] = a[vo]; pw[i] = w[vo]; pr[i] = r[vo]; pv[i] = v[vo];
-        }
-    };
-    auto form_batch = [&](int buf, uint32_t tb) {
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-            const uint32_t t = tb + 4 * wave + i;
-            if (t >= len) break;  // uniform per wave
-            const float kc = pk[i], ac = pa[i], rc = pr[i];
-            const float kk = kc * kkc_j;
-            float nrm = sqrtf(wave_sum(kk * kk));
-            nrm = nrm < eps ? eps : nrm;
-            const float kh = kk * (1.0f / nrm);
-            const float kmod = kc + ka_j * (kc * ac - kc);
-            const float bonus = wave_sum(rc * kmod * rk_j);
-            float *hv = hb[buf][4 * wave + i];
-            hv[j] = kh; hv[64 + j] = kh * (-ac); hv[128 + j] = pw[i]; hv[192 + j] = kmod; hv[256 + j] = rc; hv[320 + j] = pv[i];
-            if (j == 0) bl[buf][4 * wave + i] = bonus;
-        }
-    };
-    auto flush = [&](int buf, uint32_t tb) {
-        // kRB tokens x 64 rows = one float4 per thread (non-temporal: acknowledged sooner)
-        typedef float f4v __attribute__((ext_vector_type(4)));
-        const uint32_t u = tid >> 4, c4 = 4 * (tid & 15);
-        if (tb + u < len) {
-            const float4 yv = *(const float4 *)&yl[buf][u][c4];
-            __builtin_nontemporal_store((f4v){yv.x, yv.y, yv.z, yv.w}, (f4v *)(y_out + (size_t)(t0 + tb + u) * C + (size_t)h * 64 + c4));
-        }
-        if (tid < kRB && tb + tid < len) __builtin_nontemporal_store(bl[buf][tid], bonus_out + (size_t)(t0 + tb + tid) * H + h);
-    };
-    if (len > 0) {
-        load_batch(0);
-        form_batch(0, 0);
-    }
-    for (uint32_t tb = 0; tb < len; tb += kRB) {
-        const int buf = (tb / kRB) & 1;
-        // the batch's vectors are in LDS (lgkmcnt(0), then the barrier); the
-        // other buffer is free
-        __builtin_amdgcn_s_waitcnt(0xC07F);
-        __builtin_amdgcn_s_barrier();
-        if (tb > 0) flush(buf ^ 1, tb - kRB);  // the previous batch's outputs
-        const bool more = tb + kRB < len;
-        if (more) load_batch(tb + kRB);  // in flight during the scan below
-        const uint32_t nt = len - tb < (uint32_t)kRB ? len - tb : (uint32_t)kRB;
-        for (uint32_t u = 0; u < nt; u++) {
-            const float *hv = hb[buf][u];
-            float kv[16], bv[16], wv[16], mv[16], rv[16], vc[RPL];
-#pragma unroll
-            for (int m = 0; m < 4; m++) {
-                const float4 a0 = *(const float4 *)(hv + 16 * q + 4 * m), a1 = *(const float4 *)(hv + 64 + 16 * q + 4 * m),
-                             a2 = *(const float4 *)(hv + 128 + 16 * q + 4 * m), a3 = *(const float4 *)(hv + 192 + 16 * q + 4 * m),
-                             a4 = *(const float4 *)(hv + 256 + 16 * q + 4 * m);
-                kv[4 * m] = a0.x; kv[4 * m + 1] = a0.y; kv[4 * m + 2] = a0.z; kv[4 * m + 3] = a0.w;
-                bv[4 * m] = a1.x; bv[4 * m + 1] = a1.y; bv[4 * m + 2] = a1.z; bv[4 * m + 3] = a1.w;
-                wv[4 * m] = a2.x; wv[4 * m + 1] = a2.y; wv[4 * m + 2] = a2.z; wv[4 * m + 3] = a2.w;
-                mv[4 * m] = a3.x; mv[4 * m + 1] = a3.y; mv[4 * m + 2] = a3.z; mv[4 * m + 3] = a3.w;
-                rv[4 * m] = a4.x; rv[4 * m + 1] = a4.y; rv[4 * m + 2] = a4.z; rv[4 * m + 3] = a4.w;
-            }
-#pragma unroll
-            for (int i = 0; i < RPL; i++) vc[i] = hv[320 + row0 + i];
-            float sa[RPL], y[RPL];
-#pragma unroll
-            for (int i = 0; i < RPL; i++) {
-                sa[i] = 0.f;
-#pragma unroll
-                for (int e = 0; e < 16; e++) sa[i] = fmaf(s[i][e], kv[e], sa[i]);
-            }
-#pragma unroll
-            for (int i = 0; i < RPL; i++) sa[i] = quad_sum(sa[i]);
-#pragma unroll
-            for (int i = 0; i < RPL; i++) {
-                y[i] = 0.f;
-#pragma unroll
-                for (int e = 0; e < 16; e++) {
-                    const float ns = s[i][e] * wv[e] + sa[i] * bv[e] + vc[i] * mv[e];
-                    s[i][e] = ns;
-                    y[i] = fmaf(ns, rv[e], y[i]);
-                }
-            }
-#pragma unroll
-            for (int i = 0; i < RPL; i++) y[i] = quad_sum(y[i]);
-            if (q == 0)
-#pragma unroll
-                for (int i = 0; i < RPL; i++) yl[buf][u][row0 + i] = y[i];
-        }
-        if (more) form_batch(buf ^ 1, tb + kRB);
-    }
-    if (len > 0) {
-        __builtin_amdgcn_s_waitcnt(0xC07F);
-        __builtin_amdgcn_s_barrier();
-        const uint32_t last = (len - 1) / kRB * kRB;
-        flush((last / kRB) & 1, last);
-    }
-#pragma unroll
-    for (int i = 0; i < RPL; i++)
-#pragma unroll
-        for (int m = 0; m < 4; m++)
-            Sb[(row0 + i) * 16 + 4 * q + m] = make_float4(s[i][4 * m], s[i][4 * m + 1], s[i][4 * m + 2], s[i][4 * m + 3]);
-}
-
-// The scan for latency-bound launches (few segments: a long prompt of one
-// session, or a handful): one state row per lane group of G lanes, each lane
-// 64/G columns, G waves per (head, segment).  The dependent chain per token
-// is 64/G multiply-adds and a log2(G)-step DPP sum instead of 16 and two, at
-// G times the threads of k_wkv7_seq_rows<1>.  The head's column vectors of
-// a batch of tokens are formed into LDS one token per wave (16 per batch).
-template <int G>
-__device__ __forceinline__ float group_allsum(float v) {
-    v += quad_dpp<0xB1>(v);  // quad_perm 1,0,3,2
-    v += quad_dpp<0x4E>(v);  // quad_perm 2,3,0,1
-    if (G >= 8) v += quad_dpp<0x141>(v);   // row_half_mirror: the 8-lane sum in every lane of the 8
-    if (G >= 16) v += quad_dpp<0x140>(v);  // row_mirror: the 16-lane sum in every lane of the row
-    return v;
-}
-
-template <int G>
-__global__ __launch_bounds__(64 * G) void k_wkv7_seq_cols(
-    float *__restrict__ S, const float *__restrict__ r, const float *__restrict__ w, const float *__restrict__ k,
-    const float *__restrict__ v, const float *__restrict__ a, const float *__restrict__ kkc,
-    const float *__restrict__ ka, const float *__restrict__ rk, float *__restrict__ y_out,
-    float *__restrict__ bonus_out, const uint32_t *__restrict__ seg_start, const uint32_t *__restrict__ seg_len,
-    const uint32_t *__restrict__ seg_slot, int H, float eps, uint64_t rows, uint64_t slots) {
-    constexpr int NW = G;           // waves per (head, segment)
-    constexpr int CPL = 64 / G;     // columns per lane
-    constexpr int TPW = G >= 4 ? 1 : 4 / G;
-    constexpr int kRB = NW * TPW;   // tokens per batch
+    constexpr int G = 8;         // lanes per row, waves per (head, segment)
+    constexpr int CPL = 64 / G;  // columns per lane
+    constexpr int kRB = G;       // tokens per batch
     __shared__ __attribute__((aligned(16))) float hb[2][kRB][6 * 64];
     __shared__ __attribute__((aligned(16))) float yl[2][kRB][64];
     __shared__ float bl[2][kRB];
@@ -1028,31 +877,23 @@ __global__ __launch_bounds__(64 * G) void k_wkv7_seq_cols(
     }
     const int j = lane;
     const float kkc_j = kkc[h * 64 + j], ka_j = ka[h * 64 + j], rk_j = rk[h * 64 + j];
-    float pk[TPW], pa[TPW], pw[TPW], pr[TPW], pv[TPW];
+    float pk, pa, pw, pr, pv;
     auto load_batch = [&](uint32_t tb) {
-#pragma unroll
-        for (int i = 0; i < TPW; i++) {
-            const uint32_t t = tb + TPW * wave + i;
-            const size_t vo = (size_t)(t0 + (t < len ? t : 0)) * C + (size_t)h * 64 + j;
-            pk[i] = k[vo]; pa[i] = a[vo]; pw[i] = w[vo]; pr[i] = r[vo]; pv[i] = v[vo];
-        }
+        const uint32_t t = tb + wave;
+        const size_t vo = (size_t)(t0 + (t < len ? t : 0)) * C + (size_t)h * 64 + j;
+        pk = k[vo]; pa = a[vo]; pw = w[vo]; pr = r[vo]; pv = v[vo];
     };
     auto form_batch = [&](int buf, uint32_t tb) {
-#pragma unroll
-        for (int i = 0; i < TPW; i++) {
-            const uint32_t t = tb + TPW * wave + i;
-            if (t >= len) break;  // uniform per wave
-            const float kc = pk[i], ac = pa[i], rc = pr[i];
-            const float kk = kc * kkc_j;
-            float nrm = sqrtf(wave_sum(kk * kk));
-            nrm = nrm < eps ? eps : nrm;
-            const float kh = kk * (1.0f / nrm);
-            const float kmod = kc + ka_j * (kc * ac - kc);
-            const float bonus = wave_sum(rc * kmod * rk_j);
-            float *hv = hb[buf][TPW * wave + i];
-            hv[j] = kh; hv[64 + j] = kh * (-ac); hv[128 + j] = pw[i]; hv[192 + j] = kmod; hv[256 + j] = rc; hv[320 + j] = pv[i];
-            if (j == 0) bl[buf][TPW * wave + i] = bonus;
-        }
+        if (tb + wave >= len) return;  // uniform per wave
+        const float kk = pk * kkc_j;
+        float nrm = sqrtf(wave_sum(kk * kk));
+        nrm = nrm < eps ? eps : nrm;
+        const float kh = kk * (1.0f / nrm);
+        const float kmod = pk + ka_j * (pk * pa - pk);
+        const float bonus = wave_sum(pr * kmod * rk_j);
+        float *hv = hb[buf][wave];
+        hv[j] = kh; hv[64 + j] = kh * (-pa); hv[128 + j] = pw; hv[192 + j] = kmod; hv[256 + j] = pr; hv[320 + j] = pv;
+        if (j == 0) bl[buf][wave] = bonus;
     };
     auto flush = [&](int buf, uint32_t tb) {
         for (int e = tid; e < kRB * 64; e += 64 * G) {
@@ -1090,7 +931,7 @@ __global__ __launch_bounds__(64 * G) void k_wkv7_seq_cols(
             float sa = 0.f;
 #pragma unroll
             for (int e = 0; e < CPL; e++) sa = fmaf(s[e], kv[e], sa);
-            sa = group_allsum<G>(sa);
+            sa = oct_sum(sa);
             float y = 0.f;
 #pragma unroll
             for (int e = 0; e < CPL; e++) {
@@ -1098,7 +939,7 @@ __global__ __launch_bounds__(64 * G) void k_wkv7_seq_cols(
                 s[e] = ns;
                 y = fmaf(ns, rv[e], y);
             }
-            y = group_allsum<G>(y);
+            y = oct_sum(y);
             if (q == 0) yl[buf][u][row] = y;
         }
         if (more) form_batch(buf ^ 1, tb + kRB);
@@ -1111,6 +952,509 @@ __global__ __launch_bounds__(64 * G) void k_wkv7_seq_cols(
 #pragma unroll
     for (int m = 0; m < CPL / 4; m++)
         ((float4 *)Sr)[m] = make_float4(s[4 * m], s[4 * m + 1], s[4 * m + 2], s[4 * m + 3]);
+}
+
+// ------------------------------- chunked scan on matrix cores (fp32 MFMA)
+// The same recurrence, 16 tokens at a time.  With sigma_t the product of the
+// decays of the tokens after t in the chunk (per column; sigma_15 = 1),
+// S' = S diag(sigma_{-1}) the start state decayed to the chunk's end and
+//   kt_t = k^_t / (w_t sigma_t), rt_t = r_t / sigma_t,
+//   bh_t = -k^_t a_t sigma_t,    kh_t = k_mod_t sigma_t,
+// the step S <- S diag(w) + (S k^) b^T + v k_mod^T of every token of the
+// chunk becomes, with the rows u_t = S_{t-1} k^_t and v_t stacked as U, V,
+//   U = (I - A)^{-1} (kt S'^T + Bm V),  A_ts = bh_s.kt_t, Bm_ts = kh_s.kt_t (s < t),
+//   Y = rt S'^T + Ay U + By V,          Ay_ts = bh_s.rt_t, By_ts = kh_s.rt_t (s <= t),
+//   S_end = S' + U^T bh + V^T kh.
+// All of A, Bm, Ay, By and P = (I - A)^{-1} kt, G = (I - A)^{-1} Bm depend on
+// the inputs alone: one wave prepares one chunk (kt, rt, bh, kh with four
+// tokens x four columns a lane; the Gram products on v_mfma_f32_16x16x4_f32; P
+// and G by forward substitution, which keeps the error of the sequential order
+// where powers of A would not).  Then the state passes through the chunk as
+// U = P S'^T + G V, Y, S_end, each wave holding 16 state rows (rows are
+// independent).  Products, sums and everything kept stay fp32; the state's
+// error against 64 bits is that of the token-by-token scan (40 heads, 24
+// segments of 4096 tokens 8.5e-8 : 8.4e-8, 8 x 512 8.9e-8 : 8.4e-8).
+//   - S is held transposed in the MFMA accumulator layout: lane l, register
+//     (q, e) is S[row = l%16][column = 16q + 4(l/16) + e].  As the B operand of
+//     k-step (q, e) it is used in place: the four k of a step may be any four
+//     columns, and A's lane reads the same ones, one 16-byte LDS read per q.
+//     U's result layout (token 4(l/16) + e, row l%16) is B-operand layout too.
+//   - LDS: rows of 68 floats, read as 16 rows x one 16-byte piece, as 4 rows x 16
+//     consecutive floats and as whole rows; rt has rows of 64 with piece p of
+//     row t at p ^ t (160 KB hold eight chunks), rows of 16 keep piece p at
+//     p ^ (t/4).  All reads are free of bank conflicts.
+//   - A chunk whose Gram products pass 2^40 or are not finite (strong decays, or
+//     inputs not finite), where 0 * inf would reach the chunk's earlier tokens, is
+//     stepped token by token by the same waves, and so is one of few tokens (a
+//     decode row packed among prompts).
+constexpr int kNt = 2;  // cache policy of a buffer store: non-temporal
+constexpr int kMmLd = 68;
+struct WkvChunk {
+    float p[16 * kMmLd];    // P            (token by token: k^)
+    float rt[16 * 64];      // rt           (r)
+    float bh[16 * kMmLd];   // bh           (-k^ a)
+    float kh[16 * kMmLd];   // kh           (k_mod); [64], between rows: whether to step token by token
+    float m[3][16 * 16];    // G, Ay, By
+    float dec[64];          // sigma_{-1}
+};
+constexpr int kMmStep = 2;  // chunks of at most this many tokens are stepped token by token
+
+typedef float f4_t __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ int mm64(int t, int c) { return t * 64 + (c ^ (t << 2)); }
+__device__ __forceinline__ int mm16(int t, int s) { return t * 16 + (s ^ (t >> 2 << 2)); }
+__device__ __forceinline__ f4_t mfma4(float a, float b, f4_t c) {
+    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+}
+// 1/x to within an ulp (x normal and in range here)
+__device__ __forceinline__ float rcp_n(float x) {
+    const float y = __builtin_amdgcn_rcpf(x);
+    return fmaf(fmaf(-x, y, 1.0f), y, y);
+}
+// Sum over the four 16-lane groups, in every lane: a swap of the halves (of
+// the odd and even groups) of two copies leaves both addends in a lane.
+__device__ __forceinline__ float xsum_groups(float v) {
+    const auto p = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    v = __uint_as_float(p[0]) + __uint_as_float(p[1]);
+    const auto q = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return __uint_as_float(q[0]) + __uint_as_float(q[1]);
+}
+// LDS made visible to the block; global loads and stores stay in flight
+__device__ __forceinline__ void lds_barrier() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
+// One lane's part of a chunk in flight: tokens 4(l/16) .. +3, columns 4(l%16) .. +3.
+struct WkvTok {
+    f4_t k[4], a[4], w[4], r[4];
+};
+
+// Accesses through a buffer resource over the chunk's nt rows of one head: a
+// row past the end reads as zeros and is not written.  (The row offset goes
+// into the lane offset: the range check does not cover the scalar one.)
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t mm_rsrc(const float *p, size_t C, uint32_t nt) {
+    return __builtin_amdgcn_make_buffer_rsrc((void *)p, (short)0, nt ? (int)(((nt - 1) * C + 64) * 4) : 0, 0x00020000);
+}
+__device__ __forceinline__ float mm_ld(__amdgpu_buffer_rsrc_t rs, int off) {
+    return __int_as_float(__builtin_amdgcn_raw_buffer_load_b32(rs, off, 0, 0));
+}
+__device__ __forceinline__ f4_t mm_ld4(__amdgpu_buffer_rsrc_t rs, int off) {
+    return __builtin_bit_cast(f4_t, __builtin_amdgcn_raw_buffer_load_b128(rs, off, 0, 0));
+}
+
+__device__ __forceinline__ void mm_load(WkvTok &x, const float *__restrict__ k, const float *__restrict__ a,
+                                        const float *__restrict__ w, const float *__restrict__ r, size_t o, size_t C,
+                                        uint32_t nt, int lane) {
+    const __amdgpu_buffer_rsrc_t bk = mm_rsrc(k + o, C, nt), ba = mm_rsrc(a + o, C, nt), bw = mm_rsrc(w + o, C, nt),
+                                 br = mm_rsrc(r + o, C, nt);
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        const int o4 = ((4 * (lane >> 4) + i) * (int)C + 4 * (lane & 15)) * 4;
+        x.k[i] = mm_ld4(bk, o4); x.a[i] = mm_ld4(ba, o4); x.w[i] = mm_ld4(bw, o4); x.r[i] = mm_ld4(br, o4);
+    }
+}
+
+// The token-by-token vectors of a chunk: k^ (kk scaled by inv), r, -k^ a, k_mod.
+__device__ __forceinline__ void mm_plain(WkvChunk &c, const WkvTok &x, int lane, f4_t kkc, f4_t ka, const float (&inv)[4]) {
+    const int l16 = lane & 15, g = lane >> 4;
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        const int t = 4 * g + i, o = t * 64 + ((l16 ^ t) << 2), o2 = t * kMmLd + 4 * l16;
+        const f4_t kh = x.k[i] * kkc * inv[i];
+        *(f4_t *)&c.p[o2] = kh;
+        *(f4_t *)&c.rt[o] = x.r[i];
+        *(f4_t *)&c.bh[o2] = kh * -x.a[i];
+        *(f4_t *)&c.kh[o2] = x.k[i] + ka * (x.k[i] * x.a[i] - x.k[i]);
+    }
+}
+
+// One wave prepares one chunk of nt tokens (1..16) in LDS; returns whether it
+// is to be stepped token by token.  load(y) reads the chunk again (the rare
+// token-by-token case); fetch() reads the wave's next chunk into x.
+template <class L, class F>
+__device__ __forceinline__ int mm_prepare(WkvChunk &c, WkvTok &x, uint32_t nt, int lane, f4_t kkc, f4_t ka, f4_t rk,
+                                          float eps, float *__restrict__ bonus, int H, L load, F fetch) {
+    asm volatile("" : "+v"(lane));  // LDS addresses formed here, not kept in registers around the chunk loop
+    const int l16 = lane & 15, g = lane >> 4;
+    f4_t kk[4], km[4];
+    float bs[4], inv[4];
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        if (4 * g + i >= (int)nt) x.w[i] = (f4_t){1.0f, 1.0f, 1.0f, 1.0f};  // past the end k, a, r read as 0
+        kk[i] = x.k[i] * kkc;
+        km[i] = x.k[i] + ka * (x.k[i] * x.a[i] - x.k[i]);
+        // the head sums of the token: |kk|^2 and the bonus (a token's columns lie in one 16-lane row)
+        const f4_t q = kk[i] * kk[i], z = x.r[i] * km[i] * rk;
+        const float ss = row16_sum((q[0] + q[1]) + (q[2] + q[3]));
+        bs[i] = row16_sum((z[0] + z[1]) + (z[2] + z[3]));
+        // 1 / max(|kk|, eps): reciprocal root and one Newton step
+        const float y = __builtin_amdgcn_rsqf(ss);
+        inv[i] = ss < eps * eps ? 1.0f / eps : fmaf(0.5f * y, fmaf(-ss * y, y, 1.0f), y);
+    }
+    if (bonus && l16 < 4 && 4 * g + l16 < (int)nt)
+        __builtin_nontemporal_store(l16 == 0 ? bs[0] : l16 == 1 ? bs[1] : l16 == 2 ? bs[2] : bs[3],
+                                    bonus + (size_t)(4 * g + l16) * H);
+    // sigma of the lane's last token: the decays of the later groups' tokens
+    const f4_t pg = (x.w[0] * x.w[1]) * (x.w[2] * x.w[3]);
+    f4_t sg, rs;
+#pragma unroll
+    for (int e = 0; e < 4; e++) {
+        const auto p16 = __builtin_amdgcn_permlane16_swap(__float_as_uint(pg[e]), __float_as_uint(pg[e]), false, false);
+        const float pair = __uint_as_float(p16[0]) * __uint_as_float(p16[1]);
+        const auto p32 = __builtin_amdgcn_permlane32_swap(__float_as_uint(pair), __float_as_uint(pair), false, false);
+        sg[e] = ((g & 1) ? 1.0f : __uint_as_float(p16[1])) * (g < 2 ? __uint_as_float(p32[1]) : 1.0f);
+        rs[e] = rcp_n(sg[e]);
+    }
+#pragma unroll
+    for (int i = 3; i >= 0; i--) {
+        const int t = 4 * g + i, o = t * 64 + ((l16 ^ t) << 2), o2 = t * kMmLd + 4 * l16;
+        kk[i] *= inv[i];
+        *(f4_t *)&c.bh[o2] = kk[i] * -x.a[i] * sg;
+        *(f4_t *)&c.kh[o2] = km[i] * sg;
+        *(f4_t *)&c.rt[o] = x.r[i] * rs;
+        sg *= x.w[i];
+#pragma unroll
+        for (int e = 0; e < 4; e++) rs[e] = rcp_n(sg[e]);
+        *(f4_t *)&c.p[o2] = kk[i] * rs;
+    }
+    if (g == 0) *(f4_t *)&c.dec[4 * l16] = sg;
+    f4_t ga = {0, 0, 0, 0}, gb = ga, gy = ga, gz = ga;
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+        const int o = mm64(l16, 16 * q + 4 * g), o2 = l16 * kMmLd + 16 * q + 4 * g;
+        const f4_t kt = *(const f4_t *)&c.p[o2], rt = *(const f4_t *)&c.rt[o], bh = *(const f4_t *)&c.bh[o2],
+                   kh = *(const f4_t *)&c.kh[o2];
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            ga = mfma4(kt[e], bh[e], ga);
+            gb = mfma4(kt[e], kh[e], gb);
+            gy = mfma4(rt[e], bh[e], gy);
+            gz = mfma4(rt[e], kh[e], gz);
+        }
+    }
+    // every scaled value meets a sum here, and values out of range leave one out
+    // of range: 2^40, infinities and NaNs above it as bits
+    // (and so must the decay over the chunk be, which the state is scaled by)
+    uint32_t mag = 0;
+#pragma unroll
+    for (int e = 0; e < 4; e++)
+        mag = max(mag, max(__float_as_uint(sg[e]) & 0x7FFFFFFFu, __float_as_uint(rs[e]) & 0x7FFFFFFFu));
+#pragma unroll
+    for (int e = 0; e < 4; e++)
+        mag = max(max(max(mag, __float_as_uint(ga[e]) & 0x7FFFFFFFu), max(__float_as_uint(gb[e]) & 0x7FFFFFFFu, __float_as_uint(gy[e]) & 0x7FFFFFFFu)),
+                  __float_as_uint(gz[e]) & 0x7FFFFFFFu);
+    const bool step = __ballot(mag >= 0x53800000u) != 0 || nt <= (uint32_t)kMmStep;
+    if (step) {
+        WkvTok y;
+        load(y);
+        mm_plain(c, y, lane, kkc, ka, inv);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    fetch();
+    __builtin_amdgcn_sched_barrier(0);
+    if (step) return 1;
+    // A and Bm by row and column for the substitution
+#pragma unroll
+    for (int e = 0; e < 4; e++) {
+        const int t = 4 * g + e;
+        c.m[0][t * 16 + l16] = l16 < t ? ga[e] : 0.0f;
+        c.m[1][t * 16 + l16] = l16 < t ? gb[e] : 0.0f;
+        gy[e] = l16 <= t ? gy[e] : 0.0f;
+        gz[e] = l16 <= t ? gz[e] : 0.0f;
+    }
+    // P and G row by row (lane = column; G's 16 columns in every group), the
+    // next row of A read ahead
+    float gk[16], gg[16];
+    f4_t at[4], an[4];
+#pragma unroll
+    for (int t = 0; t < 16; t++) {
+        gk[t] = c.p[t * kMmLd + lane];
+        gg[t] = c.m[1][t * 16 + l16];
+    }
+    at[0] = *(const f4_t *)&c.m[0][16];
+#pragma unroll
+    for (int t = 1; t < 16; t++) {
+#pragma unroll
+        for (int s4 = 0; s4 < (t + 4) / 4; s4++)
+            if (t < 15) an[s4] = *(const f4_t *)&c.m[0][(t + 1) * 16 + 4 * s4];
+        float y0 = gk[t], y1 = 0.0f, z0 = gg[t], z1 = 0.0f;
+#pragma unroll
+        for (int i = 0; i < t; i++) {
+            if (i & 1) {
+                y1 = fmaf(at[i / 4][i % 4], gk[i], y1);
+                z1 = fmaf(at[i / 4][i % 4], gg[i], z1);
+            } else {
+                y0 = fmaf(at[i / 4][i % 4], gk[i], y0);
+                z0 = fmaf(at[i / 4][i % 4], gg[i], z0);
+            }
+        }
+        gk[t] = y0 + y1;
+        gg[t] = z0 + z1;
+#pragma unroll
+        for (int s4 = 0; s4 < (t + 4) / 4; s4++) at[s4] = an[s4];
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    // (the reads of m are done: LDS operations of a wave are in order)
+#pragma unroll
+    for (int t = 0; t < 16; t++) c.p[t * kMmLd + lane] = gk[t];
+    if (g == 0) {
+#pragma unroll
+        for (int t = 0; t < 16; t++) c.m[0][mm16(t, l16)] = gg[t];
+    }
+#pragma unroll
+    for (int e = 0; e < 4; e++) {
+        c.m[1][mm16(4 * g + e, l16)] = gy[e];
+        c.m[2][mm16(4 * g + e, l16)] = gz[e];
+    }
+    return 0;
+}
+
+// The operands of a chunk that its first products take, read ahead (during
+// the last products of the chunk before).
+struct WkvOps {
+    f4_t p[4], rt[4], dec[4], mg, mz;
+};
+__device__ __forceinline__ void mm_ops(WkvOps &o, const WkvChunk &c, int lane) {
+    const int l16 = lane & 15, g = lane >> 4;
+    o.mg = *(const f4_t *)&c.m[0][mm16(l16, 4 * g)];
+    o.mz = *(const f4_t *)&c.m[2][mm16(l16, 4 * g)];
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+        o.dec[q] = *(const f4_t *)&c.dec[16 * q + 4 * g];
+        o.p[q] = *(const f4_t *)&c.p[l16 * kMmLd + 16 * q + 4 * g];
+        o.rt[q] = *(const f4_t *)&c.rt[mm64(l16, 16 * q + 4 * g)];
+    }
+}
+
+// The wave's 16 state rows through one prepared chunk, whose operands o were
+// read ahead; reads those of the next chunk n.  v: this lane's values of
+// tokens 4(l/16) + e, row l%16 (0 past the end); y as v.
+__device__ __forceinline__ void mm_consume(const WkvChunk &c, const WkvChunk &n, WkvOps &o, f4_t (&s)[4], const f4_t v,
+                                           f4_t &y, int lane) {
+    const int l16 = lane & 15, g = lane >> 4;
+    // The reads of a later phase go out one after each product of the phase
+    // before it (the groups below order them): fp32 products leave a wave's issue
+    // slots to LDS reads, but not to its VALU.
+    float kh[4][4], bh[4][4];
+#pragma unroll
+    for (int e = 0; e < 4; e++)
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            kh[e][q] = c.kh[(4 * g + e) * kMmLd + 16 * q + l16];
+            bh[e][q] = c.bh[(4 * g + e) * kMmLd + 16 * q + l16];
+        }
+    const f4_t my = *(const f4_t *)&c.m[1][mm16(l16, 4 * g)];
+    // one chain of 16 columns per q, added as a tree
+    f4_t u[4], z[4];
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+        s[q] *= o.dec[q];
+        u[q] = z[q] = (f4_t){0, 0, 0, 0};
+    }
+    f4_t ug = {0, 0, 0, 0}, yz = ug;
+#pragma unroll
+    for (int e = 0; e < 4; e++) {
+        ug = mfma4(o.mg[e], v[e], ug);
+        yz = mfma4(o.mz[e], v[e], yz);
+    }
+#pragma unroll
+    for (int e = 0; e < 4; e++)
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            u[q] = mfma4(o.p[q][e], s[q][e], u[q]);
+            z[q] = mfma4(o.rt[q][e], s[q][e], z[q]);
+        }
+#pragma unroll
+    for (int i = 0; i < 40; i++) {
+        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // a product
+        __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);  // an LDS read
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    // V^T kh in sums of its own: one rounding at the state's size instead of 16
+    // (with the chain begun at S' the state's error was 1.2e-7 against 8e-8)
+    f4_t vk[4];
+#pragma unroll
+    for (int q = 0; q < 4; q++) vk[q] = (f4_t){0, 0, 0, 0};
+#pragma unroll
+    for (int e = 0; e < 4; e++)
+#pragma unroll
+        for (int q = 0; q < 4; q++) vk[q] = mfma4(kh[e][q], v[e], vk[q]);
+    const f4_t us = ((u[0] + u[1]) + (u[2] + u[3])) + ug;
+    __builtin_amdgcn_sched_barrier(0);
+    mm_ops(o, n, lane);
+#pragma unroll
+    for (int e = 0; e < 4; e++) {
+#pragma unroll
+        for (int q = 0; q < 4; q++) s[q] = mfma4(bh[e][q], us[e], s[q]);
+        yz = mfma4(my[e], us[e], yz);
+    }
+#pragma unroll
+    for (int i = 0; i < 20; i++) {
+        __builtin_amdgcn_sched_group_barrier(0x008, 1, 1);
+        __builtin_amdgcn_sched_group_barrier(0x100, 1, 1);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int q = 0; q < 4; q++) s[q] += vk[q];
+    y = ((z[0] + z[1]) + (z[2] + z[3])) + yz;
+}
+
+// The same, token by token, on the plain vectors (see WkvChunk).
+__device__ __forceinline__ void mm_step(const WkvChunk &c, f4_t (&s)[4], const f4_t v, f4_t &y, int lane,
+                                        const float *__restrict__ w, size_t C, uint32_t nt) {
+    asm volatile("" : "+v"(lane));
+    const int l16 = lane & 15, g = lane >> 4;
+    for (uint32_t t = 0; t < nt; t++) {
+        const float vt = __shfl((t & 3) == 0 ? v[0] : (t & 3) == 1 ? v[1] : (t & 3) == 2 ? v[2] : v[3], 16 * (int)(t >> 2) + l16);
+        float sa = 0.0f, yt = 0.0f;
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            const f4_t kh = *(const f4_t *)&c.p[t * kMmLd + 16 * q + 4 * g];
+#pragma unroll
+            for (int e = 0; e < 4; e++) sa = fmaf(s[q][e], kh[e], sa);
+        }
+        sa = xsum_groups(sa);
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            const int o = mm64(t, 16 * q + 4 * g);
+            const f4_t wt = *(const f4_t *)(w + t * C + 16 * q + 4 * g);
+            const f4_t b = *(const f4_t *)&c.bh[t * kMmLd + 16 * q + 4 * g], km = *(const f4_t *)&c.kh[t * kMmLd + 16 * q + 4 * g],
+                       rt = *(const f4_t *)&c.rt[o];
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                s[q][e] = s[q][e] * wt[e] + sa * b[e] + vt * km[e];
+                yt = fmaf(s[q][e], rt[e], yt);
+            }
+        }
+        yt = xsum_groups(yt);
+#pragma unroll
+        for (int e = 0; e < 4; e++) y[e] = (int)t == 4 * g + e ? yt : y[e];
+    }
+}
+
+// One block per (head, segment, 4/NC-th of its rows): waves NC.. prepare the
+// next NP chunks, one each, into one set while waves 0..NC-1 pass the state's
+// rows, 16 each, through the NP chunks of the other.
+//   <4, 4>: the preparing is done once per head; 8 waves, one block per CU.
+//   <1, 3>: a quarter of the rows per block, for launches that leave CUs idle.
+//     fp32 MFMA holds its SIMD's VALU for half of its 32 cycles, so a preparing
+//     wave beside a passing one slows both; here each has a SIMD of its own.
+template <int NC, int NP>
+__global__ __launch_bounds__(64 * (NC + NP), (NC + NP) / 4) void k_wkv7_seq_mm(
+    float *__restrict__ S, const float *__restrict__ r, const float *__restrict__ w, const float *__restrict__ k,
+    const float *__restrict__ v, const float *__restrict__ a, const float *__restrict__ kkc,
+    const float *__restrict__ ka, const float *__restrict__ rk, float *__restrict__ y_out,
+    float *__restrict__ bonus_out, const uint32_t *__restrict__ seg_start, const uint32_t *__restrict__ seg_len,
+    const uint32_t *__restrict__ seg_slot, int H, float eps, uint64_t rows, uint64_t slots) {
+    __shared__ __attribute__((aligned(16))) WkvChunk chunk[2][NP];
+    constexpr uint32_t kSup = 16 * NP;  // tokens of a superstep
+    const int h = blockIdx.x, gi = blockIdx.y, tid = threadIdx.x;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, l16 = lane & 15, g = lane >> 4;
+    const size_t C = (size_t)H * 64;
+    const uint32_t t0 = seg_start[gi], len = seg_len[gi], slot = seg_slot[gi];
+    if (slot >= slots || (uint64_t)t0 + len > rows || len == 0) return;  // uniform per block
+    const uint32_t nsup = (len + kSup - 1) / kSup;
+    const size_t col = (size_t)t0 * C + (size_t)h * 64;
+    auto ntok = [&](uint32_t tb) -> uint32_t { return tb < len ? (len - tb < 16 ? len - tb : 16) : 0; };
+    // both roles meet nsup times: superstep i is in LDS at the i-th meeting,
+    // and superstep i-1 has been passed through
+    if (wave >= NC) {
+        const f4_t kkc_j = *(const f4_t *)(kkc + h * 64 + 4 * l16), ka_j = *(const f4_t *)(ka + h * 64 + 4 * l16),
+                   rk_j = *(const f4_t *)(rk + h * 64 + 4 * l16);
+        const int pw = wave - NC;
+        WkvTok x;
+        auto load = [&](WkvTok &y, uint32_t tb) { mm_load(y, k, a, w, r, col + (size_t)tb * C, C, ntok(tb), lane); };
+        load(x, 16 * pw);
+        for (uint32_t sup = 0; sup < nsup; sup++) {
+            const uint32_t tb = kSup * sup + 16 * pw, nt = ntok(tb);
+            if (nt) {
+                float *bonus = blockIdx.z == 0 ? bonus_out + (size_t)(t0 + tb) * H + h : nullptr;
+                WkvChunk &c = chunk[sup & 1][pw];
+                const int st = mm_prepare(c, x, nt, lane, kkc_j, ka_j, rk_j, eps, bonus, H,
+                                          [&](WkvTok &y) { load(y, tb); }, [&] { load(x, tb + kSup); });
+                if (lane == 0) c.kh[64] = __int_as_float(st);
+            }
+            lds_barrier();
+        }
+        return;
+    }
+    const int pw = NC * blockIdx.z + wave;  // this wave's rows: 16 pw ..
+    float *Srow = S + ((size_t)slot * H + h) * 4096 + (size_t)(16 * pw + l16) * 64;
+    // v of a superstep's chunks, a superstep ahead
+    auto vload = [&](f4_t (&z)[NP], uint32_t tb) {
+#pragma unroll
+        for (int i = 0; i < NP; i++) {
+            const __amdgpu_buffer_rsrc_t bv = mm_rsrc(v + col + (size_t)(tb + 16 * i) * C, C, ntok(tb + 16 * i));
+#pragma unroll
+            for (int e = 0; e < 4; e++) z[i][e] = mm_ld(bv, ((4 * g + e) * (int)C + 16 * pw + l16) * 4);
+        }
+    };
+    f4_t s[4];
+#pragma unroll
+    for (int q = 0; q < 4; q++) s[q] = *(const f4_t *)(Srow + 16 * q + 4 * g);
+    f4_t vn[NP];
+    vload(vn, 0);
+    for (uint32_t sup = 0; sup < nsup; sup++) {
+        const int set = sup & 1;
+        lds_barrier();
+        WkvOps o;
+        const int stepped = __float_as_int(chunk[set][lane < NP ? lane : 0].kh[64]);
+        mm_ops(o, chunk[set][0], lane);
+        f4_t vs[NP];
+#pragma unroll
+        for (int i = 0; i < NP; i++) vs[i] = vn[i];
+        vload(vn, kSup * (sup + 1));
+#pragma unroll 1
+        for (int i = 0; i < NP; i++) {
+            const uint32_t tb = kSup * sup + 16 * i, nt = ntok(tb);
+            if (!nt) break;
+            f4_t vc = vs[0], y;
+#pragma unroll
+            for (int j = 0; j < NP - 1; j++) vs[j] = vs[j + 1];
+            // a value of v that is not finite stays out of the products (0 * inf
+            // would reach earlier tokens) and is put on the row's later tokens
+            // and state below
+            const bool poison = __ballot(!((fabsf(vc[0]) + fabsf(vc[1])) + (fabsf(vc[2]) + fabsf(vc[3])) <= 3.4028235e38f)) != 0;
+            const f4_t vraw = vc;
+            if (poison) {
+#pragma unroll
+                for (int e = 0; e < 4; e++) vc[e] = fabsf(vc[e]) <= 3.4028235e38f ? vc[e] : 0.0f;
+            }
+            const WkvChunk &next = chunk[set][i < NP - 1 ? i + 1 : i];
+            if (__builtin_amdgcn_readlane(stepped, i)) {
+                mm_step(chunk[set][i], s, vc, y, lane, w + col + (size_t)tb * C, C, nt);
+                mm_ops(o, next, lane);
+            } else {
+                mm_consume(chunk[set][i], next, o, s, vc, y, lane);
+            }
+            if (poison) {
+                int first = 16;  // the row's first such token
+#pragma unroll
+                for (int e = 3; e >= 0; e--) first = fabsf(vraw[e]) <= 3.4028235e38f ? first : 4 * g + e;
+                first = min(first, __shfl_xor(first, 16));
+                first = min(first, __shfl_xor(first, 32));
+#pragma unroll
+                for (int e = 0; e < 4; e++) y[e] = 4 * g + e >= first ? __builtin_nanf("") : y[e];
+#pragma unroll
+                for (int q = 0; q < 4; q++)
+#pragma unroll
+                    for (int e = 0; e < 4; e++) s[q][e] = first < 16 ? __builtin_nanf("") : s[q][e];
+            }
+            // wait for the next superstep's v here: after these stores the wait
+            // would be for them too
+            if (i == NP - 1) {
+#pragma unroll
+                for (int j = 0; j < NP; j++) asm volatile("" : "+v"(vn[j]));
+            }
+            const __amdgpu_buffer_rsrc_t by = mm_rsrc(y_out + col + (size_t)tb * C, C, nt);
+#pragma unroll
+            for (int e = 0; e < 4; e++)
+                __builtin_amdgcn_raw_buffer_store_b32(__float_as_int(y[e]), by, ((4 * g + e) * (int)C + 16 * pw + l16) * 4, 0, kNt);
+        }
+    }
+#pragma unroll
+    for (int q = 0; q < 4; q++) *(f4_t *)(Srow + 16 * q + 4 * g) = s[q];
 }
 
 // yg = ((GroupNorm(y) * gamma + beta) + bonus * v) * g in fp16: 16 lanes per
@@ -1151,33 +1495,29 @@ int launch_wkv7_seq_ragged_gate(rsv_ctx *ctx, float *s, const float *r, const fl
     if (n != 64) return RSV_FAIL("wkv7_seq: head_size must be 64 (got %d)", n);
     if (nseg <= 0 || rows == 0) return 0;
     {
-        // two rows per lane group (two waves per head and segment, half the
-        // LDS vector reads per state element): faster than one row (four
-        // waves) at every chunk shape of a 64-session ragged prefill, including
-        // chunks of few long segments (115.5k against 114.9k tok/s when one
-        // row per group was used below 51 segments)
-#define WKV_ROWS_LAUNCH(R)                                                                                            \
-    hipLaunchKernelGGL(k_wkv7_seq_rows<R>, dim3(h, nseg), dim3(256 / (R)), 0, ctx->stream, s, r, w, k, v, a, kk, ka, rk, \
-                       y_work, bonus_work, seg_start, seg_len, seg_slot, h, 1e-12f, rows, slots)
-#define WKV_COLS_LAUNCH(G)                                                                                            \
-    hipLaunchKernelGGL(k_wkv7_seq_cols<G>, dim3(h, nseg), dim3(64 * (G)), 0, ctx->stream, s, r, w, k, v, a, kk, ka, rk, \
-                       y_work, bonus_work, seg_start, seg_len, seg_slot, h, 1e-12f, rows, slots)
-        // (head, segment) blocks: with fewer than one per CU the launch is
-        // the longest segment's dependent chain, shortened by more lanes per row
+#define WKV_MM_LAUNCH(NC, NP)                                                                                         \
+    hipLaunchKernelGGL((k_wkv7_seq_mm<NC, NP>), dim3(h, nseg, 4 / (NC)), dim3(64 * ((NC) + (NP))), 0, ctx->stream, s, r, \
+                       w, k, v, a, kk, ka, rk, y_work, bonus_work, seg_start, seg_len, seg_slot, h, 1e-12f, rows, slots)
+        // The chunked scan from 24 tokens a segment on (the mean: the lengths are
+        // on the device), from 48 where the blocks take more than two rounds over
+        // the CUs (one block per CU; k_wkv7_seq_cols packs several).  40 heads,
+        // scan and GroupNorm pass, us against the token-by-token form taken for
+        // the shape before: 1 x 700 tokens 96 : 219, 8 x 512 191 : 448, 24
+        // segments of 4096 178 : 287, 64 of 4096 206 : 236, 32 x 512 600 : 837.
+        // Near the line, against k_wkv7_seq_cols: 1 x 40 16 : 19, 10 x 32 28 : 33,
+        // 5 x 20 16 : 16, 10 x 16 25 : 21; 24 x 43 63 : 60, 64 x 32 133 : 115.
+        // A quarter of a head's rows per block while every block still has a CU:
+        // 1 x 700 96 against 109.  RSV_SCAN_G selects a form: 4 and 1 heads per
+        // whole or quarter block, anything else token by token.
         const int blocks = h * nseg, cus = ctx->sm_count > 0 ? ctx->sm_count : 256;
         const char *e = getenv("RSV_SCAN_G");
-        // From 16 blocks per CU (e.g. 256 sessions x 40 heads) four rows per
-        // group (one wave per block, half the LDS vector reads per state
-        // element again) keeps every SIMD busy: B=256 x T=512 5.09 -> 4.68 ms;
-        // below that it leaves SIMDs idle (64 x 64 tokens: 192 -> 208 us)
-        const int gsel = e ? atoi(e)
-                           : (blocks * 4 <= cus ? 16 : blocks <= cus ? 8 : blocks >= 16 * cus ? -4 : 0);
-        if (gsel == 16) WKV_COLS_LAUNCH(16);
-        else if (gsel == 8) WKV_COLS_LAUNCH(8);
-        else if (gsel == -4) WKV_ROWS_LAUNCH(4);
-        else WKV_ROWS_LAUNCH(2);
-#undef WKV_COLS_LAUNCH
-#undef WKV_ROWS_LAUNCH
+        const int gsel = e ? atoi(e) : rows < (blocks <= 2 * cus ? 24u : 48u) * (uint64_t)nseg ? 0 : blocks * 4 <= cus ? 1 : 4;
+        if (gsel == 4) WKV_MM_LAUNCH(4, 4);
+        else if (gsel == 1) WKV_MM_LAUNCH(1, 3);
+        else
+            hipLaunchKernelGGL(k_wkv7_seq_cols, dim3(h, nseg), dim3(512), 0, ctx->stream, s, r, w, k, v, a, kk, ka, rk, y_work,
+                               bonus_work, seg_start, seg_len, seg_slot, h, 1e-12f, rows, slots);
+#undef WKV_MM_LAUNCH
         const uint64_t units = rows * (uint64_t)h;
         hipLaunchKernelGGL(k_gn_gate_f16, dim3((unsigned)((units + 15) / 16)), dim3(256), 0, ctx->stream, y_work,
                            bonus_work, v, gamma, beta, g, yg, units, h, gn_eps);

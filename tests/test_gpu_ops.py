@@ -365,6 +365,54 @@ def test_wkv7_seq_ragged_gate_matches_scan_times_gate(be, lens, scan_g, monkeypa
     assert rel_err(be.get(S2, S.size), be.get(S1, S.size)) < 1e-5
 
 
+@pytest.mark.parametrize("form", ["4", "1"])
+@pytest.mark.parametrize("kind", ["model", "strong", "big", "nan_k", "inf_v"])
+def test_wkv7_seq_chunked_matches_token_by_token(be, kind, form, monkeypatch):
+    """The chunked scan (whole heads and quarters per block) against the
+    token-by-token form, at segment lengths around its chunks of 16 and its
+    supersteps of 48 and 64 tokens: decays of the model, decays down to 0 and
+    keys of 1e13 (both leave its range and are stepped token by token), and
+    inputs that are not finite, which must reach the same tokens and rows.
+    The two sum in another order: a few hundred roundings of 2^-24 (state), a
+    16-bit output (yg)."""
+    rsv = _rsv()
+    H = 3
+    C = H * 64
+    lens = [1, 2, 3, 15, 16, 17, 33, 47, 48, 49, 63, 64, 65, 130]
+    rng = np.random.default_rng(len(kind))
+    T = sum(lens)
+    r, v, k, w, a, _, kk, ka, rk, gam, bet = _wkv_inputs(rng, T, H)
+    if kind == "strong":
+        w = rng.random((T, C)).astype(np.float32) ** 4
+        w[rng.random((T, C)) < 0.02] = 0.0
+    elif kind == "big":
+        k, rk = k * np.float32(1e13), rk * 0  # (no bonus: it would leave fp16's range)
+    elif kind == "nan_k":
+        k[T - 60, 70] = np.nan  # head 1 of the last segment
+    elif kind == "inf_v":
+        v[T - 60, 130] = np.inf  # one state row of head 2
+    g = rng.random((T, C)).astype(np.float32)
+    n = len(lens)
+    S = (rng.standard_normal((n, H, 64, 64)) * 0.1).astype(np.float32)
+    st = be.tensor(np.concatenate([[0], np.cumsum(lens)[:-1]]).astype(np.uint32), dtype=rsv.U32)
+    ln = be.tensor(np.array(lens, np.uint32), dtype=rsv.U32)
+    sl = be.tensor(np.arange(n, dtype=np.uint32)[::-1].copy(), dtype=rsv.U32)
+    common = [be.tensor(x) for x in (r, w, k, v, a, kk, ka, rk, gam, bet)]
+    out = []
+    for which in ("0", form):
+        monkeypatch.setenv("RSV_SCAN_G", which)
+        s2, gt, yw, bw = be.tensor(S), be.tensor(g), be.tensor(n=T * C), be.tensor(n=T * H)
+        yg = be.tensor(n=T * C, dtype=rsv.F16)
+        be.call("rsv_wkv7_seq_ragged_gate", s2, *common, gt, yw, bw, yg, st, ln, sl, n, T, H, 64, 64e-5)
+        out.append((be.get(yg, T * C), be.get(s2, S.size)))
+    for (got, want), tol in zip(zip(out[1], out[0]), (2e-3, 1e-5)):
+        fine = np.isfinite(want)
+        if kind in ("nan_k", "inf_v"):
+            assert not fine.all()
+        assert np.array_equal(fine, np.isfinite(got))
+        assert rel_err(got[fine], want[fine]) < tol
+
+
 @pytest.mark.parametrize("nseg", [32, 256])
 def test_wkv7_seq_config2_t512(be, nseg):
     """configs[2] at B=32 and B=256 x T=512: nseg segments of 512 tokens

@@ -498,7 +498,9 @@ int rsv_lane_select(rsv_ctx *ctx, int lane);
 int rsv_lane_record(rsv_ctx *ctx, int ev);
 int rsv_lane_wait(rsv_ctx *ctx, int lane, int ev);
 
-/* ---- raw access for harnesses: device pointer and stream of a tensor/ctx */
+/* ---- raw access for harnesses: device pointer and stream of a tensor/ctx.
+ * rsv_tensor_ptr waits for the context's stream (outside graph capture), so
+ * that a new tensor's zero fill cannot land on what another stream writes. */
 int rsv_tensor_ptr(rsv_ctx *ctx, uint32_t id, void **ptr);
 int rsv_stream(rsv_ctx *ctx, void **stream);
 

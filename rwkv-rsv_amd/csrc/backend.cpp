@@ -283,6 +283,9 @@ int rsv_tensor_len(rsv_ctx *ctx, uint32_t id, uint64_t *len, int *dtype) {
 int rsv_tensor_ptr(rsv_ctx *ctx, uint32_t id, void **ptr) {
     Tensor *t = get_tensor(ctx, id);
     if (!t) return RSV_FAIL("tensor_ptr: unknown tensor id %u", id);
+    // a new tensor's zero fill is on the context's stream: done before another
+    // stream (the pointer's likely user) can write the tensor
+    if (!ctx->capturing && !ctx->prefill_capturing) RSV_HIP(hipStreamSynchronize(ctx->stream));
     *ptr = t->ptr;
     return 0;
 }

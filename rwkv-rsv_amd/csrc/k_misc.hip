@@ -663,47 +663,115 @@ __device__ __forceinline__ void ln_pair(float (&a)[kLnVec], float (&b)[kLnVec], 
 
 struct HOut6 { _Float16 *p[6]; };
 
-__global__ __launch_bounds__(1024) void k_seq_norm_mix(const float *__restrict__ x, const float *__restrict__ state,
-                                                       const float *__restrict__ gamma, const float *__restrict__ beta,
-                                                       Ptr6 coef, HOut6 out, int nout,
-                                                       const uint32_t *__restrict__ row_prev, int C, uint64_t slots,
-                                                       float eps) {
-    __shared__ float2 red[16];
-    const int t = blockIdx.x, c0 = threadIdx.x * kLnVec;
+// Sums of v[0 .. N-1] over the block, in the order of block_sum2.  red is used
+// once (no second barrier).
+template <int N>
+__device__ __forceinline__ void block_sums(float (&v)[N], float (*red)[N]) {
+#pragma unroll
+    for (int i = 0; i < N; i++) v[i] = wave_sum_last(v[i]);
+    const int nw = blockDim.x >> 6;
+    if ((threadIdx.x & 63) == 63) {
+#pragma unroll
+        for (int i = 0; i < N; i++) red[threadIdx.x >> 6][i] = v[i];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < N; i++) v[i] = red[0][i];
+    for (int w = 1; w < nw; w++)
+#pragma unroll
+        for (int i = 0; i < N; i++) v[i] += red[w][i];
+}
+
+// R consecutive token rows per block: the row before the first and the R rows
+// are loaded at entry and their statistics taken together (two barriers a
+// block, where one pair of sums after another took four), so with R = 2 a row is
+// normalised once where its successor is in the block, and gamma, beta and the
+// mix coefficients are read once for both.  Rows of 2560 with one output: 4096
+// rows 30 -> 20 us (63 MB), 1500 12.8 -> 7.4, 700 6.5 -> 5.5; with six: 4096 43
+// -> 37 us (168 MB, 4.5 TB/s), 1500 19.6 -> 14.4, 700 10.5 -> 9.1.
+template <int R, int NT>
+__global__ __launch_bounds__(NT) void k_seq_norm_mix(const float *__restrict__ x, const float *__restrict__ state,
+                                                     const float *__restrict__ gamma, const float *__restrict__ beta,
+                                                     Ptr6 coef, HOut6 out, int nout, const uint32_t *__restrict__ row_prev,
+                                                     int T, int C, uint64_t slots, float eps) {
+    __shared__ float red[2][16][R + 1];
+    __shared__ float2 red2[16];
+    const int t0 = blockIdx.x * R, n = min(R, T - t0), c0 = threadIdx.x * kLnVec;
     const bool live = c0 < C;
-    const uint32_t p = row_prev[t];
-    const bool from_state = (p & 0x80000000u) != 0;
-    const uint32_t slot = p & 0x7FFFFFFFu;
-    // every load first: this row, its predecessor (raw x, or the LN'd state
-    // row), gamma / beta and the mix coefficients
-    float xa[kLnVec] = {}, xb[kLnVec] = {}, gm[kLnVec] = {}, bt[kLnVec] = {}, cf[6][kLnVec];
+    uint32_t p[R];
+#pragma unroll
+    for (int i = 0; i < R; i++) p[i] = row_prev[min(t0 + i, T - 1)];
+    // v[0]: the row before row t0 (raw x, or the slot's LN'd state row), v[1 + i]: row t0 + i
+    const bool first_state = (p[0] & 0x80000000u) != 0;
+    float v[R + 1][kLnVec] = {}, gm[kLnVec] = {}, bt[kLnVec] = {};
     if (live) {
-        ld8(x + (size_t)t * C + c0, xa);
-        if (!from_state) ld8(x + (size_t)p * C + c0, xb);
-        else if (slot < slots) ld8(state + (size_t)slot * C + c0, xb);
+        if (!first_state) ld8(x + (size_t)p[0] * C + c0, v[0]);
+        else if ((p[0] & 0x7FFFFFFFu) < slots) ld8(state + (size_t)(p[0] & 0x7FFFFFFFu) * C + c0, v[0]);
+#pragma unroll
+        for (int i = 0; i < R; i++) ld8(x + (size_t)min(t0 + i, T - 1) * C + c0, v[1 + i]);
         ld8(gamma + c0, gm);
         ld8(beta + c0, bt);
-#pragma unroll
-        for (int j = 0; j < 6; j++)
-            if (j < nout) ld8(coef.p[j] + c0, cf[j]);
     }
-    float pv[kLnVec];
+    float s[R + 1], q[R + 1];
 #pragma unroll
-    for (int e = 0; e < kLnVec; e++) pv[e] = xb[e];
-    ln_pair(xa, xb, gm, bt, live, C, eps, red);  // uniform per block: the barriers inside
-    if (!from_state) {
+    for (int i = 0; i <= R; i++) {
+        s[i] = q[i] = 0.0f;
 #pragma unroll
-        for (int e = 0; e < kLnVec; e++) pv[e] = xb[e];
+        for (int e = 0; e < kLnVec; e++) s[i] += v[i][e];
     }
-    if (!live) return;
+    block_sums(s, red[0]);
 #pragma unroll
-    for (int j = 0; j < 6; j++) {
-        if (j >= nout) break;
-        typedef _Float16 h8 __attribute__((ext_vector_type(8)));
-        h8 o;
+    for (int i = 0; i <= R; i++) {
+        s[i] = s[i] / (float)C;
+        if (live) {
 #pragma unroll
-        for (int e = 0; e < kLnVec; e++) o[e] = (_Float16)(xa[e] + cf[j][e] * (pv[e] - xa[e]));
-        *(h8 *)(out.p[j] + (size_t)t * C + c0) = o;
+            for (int e = 0; e < kLnVec; e++) {
+                const float d = v[i][e] - s[i];
+                q[i] += d * d;
+            }
+        }
+    }
+    block_sums(q, red[1]);
+#pragma unroll
+    for (int i = 0; i <= R; i++) {
+        if (i == 0 && first_state) continue;
+        const float inv = 1.0f / sqrtf(q[i] / (float)C + eps);
+#pragma unroll
+        for (int e = 0; e < kLnVec; e++) v[i][e] = (v[i][e] - s[i]) * inv * gm[e] + bt[e];
+    }
+    // rows whose predecessor is another one than the row before them (a
+    // segment's first row: the state; any other row of x is normalised here)
+    float alt[kLnVec];
+#pragma unroll
+    for (int i = 0; i < R; i++) {
+        const bool other = i > 0 && i < n && p[i] != (uint32_t)(t0 + i - 1);  // uniform per block
+        if (other) {
+#pragma unroll
+            for (int e = 0; e < kLnVec; e++) alt[e] = 0.0f;
+            const uint32_t slot = p[i] & 0x7FFFFFFFu;
+            if (p[i] & 0x80000000u) {
+                if (live && slot < slots) ld8(state + (size_t)slot * C + c0, alt);
+            } else {
+                float none[kLnVec] = {};
+                if (live) ld8(x + (size_t)p[i] * C + c0, alt);
+                ln_pair(alt, none, gm, bt, live, C, eps, red2);
+            }
+        }
+        if (!live || i >= n) continue;
+#pragma unroll
+        for (int j = 0; j < 6; j++) {
+            if (j >= nout) break;
+            float cf[kLnVec];
+            ld8(coef.p[j] + c0, cf);
+            typedef _Float16 h8 __attribute__((ext_vector_type(8)));
+            h8 o;
+#pragma unroll
+            for (int e = 0; e < kLnVec; e++) {
+                const float a = v[1 + i][e], b = other ? alt[e] : v[i][e];
+                o[e] = (_Float16)(a + cf[e] * (b - a));
+            }
+            *(h8 *)(out.p[j] + (size_t)(t0 + i) * C + c0) = o;
+        }
     }
 }
 
@@ -718,8 +786,16 @@ int launch_seq_norm_mix(rsv_ctx *ctx, const float *x, const float *state, const 
     Ptr6 cp{};
     HOut6 op{};
     for (int j = 0; j < nout; j++) { cp.p[j] = coef[j]; op.p[j] = out[j]; }
-    hipLaunchKernelGGL(k_seq_norm_mix, dim3(t), dim3(ln_threads(c)), 0, ctx->stream, x, state, gamma, beta, cp, op, nout,
-                       row_prev, c, slots, eps);
+    const int nt = ln_threads(c), cus = ctx->sm_count > 0 ? ctx->sm_count : 256;
+#define SNM_LAUNCH(R, NT)                                                                                             \
+    hipLaunchKernelGGL((k_seq_norm_mix<R, NT>), dim3((t + (R) - 1) / (R)), dim3(nt), 0, ctx->stream, x, state, gamma, \
+                       beta, cp, op, nout, row_prev, t, c, slots, eps)
+    // two rows a block from four rows per CU on (1500 rows of 2560, one output,
+    // 8.9 us with one and 7.4 with two; 700 rows 5.5 and 5.7; four rows a block
+    // gained nothing at 4096 and lost below)
+    if (nt <= 512 && t >= 4 * cus) SNM_LAUNCH(2, 512);
+    else SNM_LAUNCH(1, 1024);
+#undef SNM_LAUNCH
     RSV_HIP(hipGetLastError());
     return 0;
 }

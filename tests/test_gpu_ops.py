@@ -365,6 +365,41 @@ def test_wkv7_seq_ragged_gate_matches_scan_times_gate(be, lens, scan_g, monkeypa
     assert rel_err(be.get(S2, S.size), be.get(S1, S.size)) < 1e-5
 
 
+@pytest.mark.parametrize("T,c,nout", [(1, 264, 1), (1023, 264, 6), (1024, 264, 1), (1027, 264, 6), (1030, 8192, 1)])
+def test_seq_norm_mix_rows(be, T, c, nout):
+    """rsv_seq_norm_mix below and from the row count where a block takes two
+    rows: an odd last row, segments that start on a block's first and second
+    row (from a state slot, one of them out of range: zeros), and a row whose
+    predecessor is some other row.  fp16 outputs: 2^-11 relative, plus the LN's
+    fp32 sums."""
+    rsv = _rsv()
+    rng = np.random.default_rng(T + c)
+    x = (rng.standard_normal((T, c)) * 2 + 0.5).astype(np.float32)
+    state = rng.standard_normal((3, c)).astype(np.float32)
+    gam, bet = rng.standard_normal(c).astype(np.float32), rng.standard_normal(c).astype(np.float32)
+    coef = rng.random((nout, c)).astype(np.float32)
+    prev = np.arange(T, dtype=np.int64) - 1
+    prev[0] = 0x80000000 + 1
+    for row, p in ((6, 0x80000000), (13, 0x80000002), (20, 0x80000000 + 7), (31, 3), (40, 17)):
+        if row < T:
+            prev[row] = p
+    ln = lambda a: ((a - a.mean(-1, keepdims=True)) / np.sqrt(a.var(-1, keepdims=True) + 1e-5)) * gam + bet  # noqa: E731
+    L = ln(x.astype(np.float64))
+    P = np.empty_like(L)
+    for t in range(T):
+        s = prev[t] - 0x80000000
+        P[t] = L[prev[t]] if s < 0 else state[s] if s < 3 else 0.0
+    outs = [be.tensor(n=T * c, dtype=rsv.F16) for _ in range(nout)]
+    ids = [be.tensor(v) for v in (x, state, gam, bet)]
+    cid = (ctypes.c_uint32 * nout)(*[be.tensor(v) for v in coef])
+    oid = (ctypes.c_uint32 * nout)(*outs)
+    be.call("rsv_seq_norm_mix", *ids, cid, oid, nout, be.tensor(prev.astype(np.uint32), dtype=rsv.U32), T, c, 1e-5)
+    for j in range(nout):
+        want = L + coef[j] * (P - L)
+        got = be.get(outs[j], T * c).reshape(T, c)
+        assert np.all(np.abs(got - want) <= 2.0 ** -11 * np.abs(want) + 2e-5)
+
+
 @pytest.mark.parametrize("form", ["4", "1"])
 @pytest.mark.parametrize("kind", ["model", "strong", "big", "nan_k", "inf_v"])
 def test_wkv7_seq_chunked_matches_token_by_token(be, kind, form, monkeypatch):

@@ -462,8 +462,9 @@ __global__ __launch_bounds__(256, BKT == 64 ? 3 : 2) void k_gemm3_multi(GemmJobs
 // per SIMD, and the operand tiles copied global -> LDS by
 // global_load_lds_dwordx4 (no VGPR staging, no LDS stores by the waves).
 //   - A stage is 64 k of the block's BMR activation rows and BNC weight
-//     rows, 128 bytes per row; NS = 3 stages rotate, the copy of stage s+2
-//     in flight while stage s is multiplied out, one barrier per stage.
+//     rows, 128 bytes per row; NS stages rotate (3, 5 for the tiles whose
+//     stages are small), the copies of up to stage s + NS - 1 in flight while
+//     stage s is multiplied out, one barrier per stage.
 //   - Copy instruction i of wave w fills 1 KiB: rows 8g .. 8g+7 of the
 //     stage (g = w*NI + i; A rows first, then B rows), lane l taking row
 //     8g + l/8 and 16-byte piece (l%8) ^ gd_swz(row).  The XOR spreads the
@@ -472,7 +473,12 @@ __global__ __launch_bounds__(256, BKT == 64 ? 3 : 2) void k_gemm3_multi(GemmJobs
 //     blocks; per 16 k it reads MI + NJ operand pieces (ds_read_b128, in asm:
 //     the compiler cannot see which LDS copy a read waits for and would drain
 //     every copy in flight before it) and issues MI*NJ MFMAs, the reads of
-//     the next 16 k in flight during them.
+//     a later 16 k in flight during them.
+//   - What bounds it: the large tiles, with the chip full, the matrix pipes at
+//     the clock the power leaves (256x160 at 4096 x 10240 x 2560: 1020
+//     TFLOP/s); the small ones a CU's copy rate from L2 to LDS (about 80 GB/s
+//     a CU: 0.5 us a stage of 32 KB while its MFMAs take 0.25), so what does
+//     not fill the chip wants more and smaller tiles, down to 64x64.
 //   - The MFMA is the one of k_gemm2/3 (v_mfma_f32_32x32x16_f16, lane l
 //     holding k 8*(l/32) .. +7 of each 16 k, ascending k): every element's
 //     accumulation chain is the same, so the results equal the other forms'
@@ -487,8 +493,12 @@ struct GdCfg {
     static constexpr int ROWS = BMR + BNC;
     static constexpr int SB = ROWS * 128;     // bytes of one stage
     static constexpr int NI = ROWS / 8 / 4;   // copy instructions per wave per stage
-    static constexpr int NS = 3;
+    static constexpr int NS = SB <= 32 * 1024 ? 5 : 3;  // stage buffers (160 KB of LDS)
     static constexpr int LDS = NS * SB;
+    // operands are read D 16-k steps ahead: a step of at most 4 MFMAs (128
+    // cycles) does not cover the reads' latency (1000 x 768 x 768, 128x128
+    // tiles: 9.5 -> 8.9 us); 2 needs a stage more in flight than 3 buffers hold
+    static constexpr int D = NS >= 4 ? 2 : 1;
     static_assert(ROWS % 32 == 0, "stage rows must split evenly over 4 waves");
     static_assert(LDS <= 160 * 1024, "LDS");
 };
@@ -546,8 +556,7 @@ __device__ __forceinline__ void gemmd_body(const GemmArgs &g, int m0, int n0, un
     // copies row group gi = wave*NI + i: A rows 8*gi .. if gi < BMR/8, else
     // B rows 8*gi - BMR ..; lane l takes row 8*gi + l/8 and logical piece
     // (l%8) ^ gd_swz(row).
-    const __amdgpu_buffer_rsrc_t rsA = __builtin_amdgcn_make_buffer_rsrc((void *)g.a, (short)0, g.m * g.lda * 2, 0x00020000);
-    const __amdgpu_buffer_rsrc_t rsB = __builtin_amdgcn_make_buffer_rsrc((void *)g.b, (short)0, g.n * g.k * 2, 0x00020000);
+    const int sizeA = g.m * g.lda * 2, sizeB = g.n * g.k * 2, nst = g.k / 64;
     const int lr = lane >> 3;
     uint32_t voff[NI];
 #pragma unroll
@@ -558,12 +567,16 @@ __device__ __forceinline__ void gemmd_body(const GemmArgs &g, int m0, int n0, un
                              : ((uint32_t)(n0 + r - C::BMR + lr) * (uint32_t)g.k + lp * 8) * 2u;
     }
     const int nA = min(max(C::BMR / 8 - wave * NI, 0), NI);  // this wave's A instructions
+    auto copy = [&](__amdgpu_buffer_rsrc_t cA, __amdgpu_buffer_rsrc_t cB, int s, unsigned char *dst, int i) {
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(i < nA ? cA : cB, (__attribute__((address_space(3))) void *)(dst + i * 1024),
+                                                 16, voff[i], s * 128, 0, 0);
+    };
     auto issue = [&](int s, int buf) {
-        unsigned char *dst = lds + buf * C::SB + wave * NI * 1024;
+        const bool live = s < nst;
+        const __amdgpu_buffer_rsrc_t cA = __builtin_amdgcn_make_buffer_rsrc((void *)g.a, (short)0, live ? sizeA : 0, 0x00020000);
+        const __amdgpu_buffer_rsrc_t cB = __builtin_amdgcn_make_buffer_rsrc((void *)g.b, (short)0, live ? sizeB : 0, 0x00020000);
 #pragma unroll
-        for (int i = 0; i < NI; i++)
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(i < nA ? rsA : rsB, (__attribute__((address_space(3))) void *)(dst + i * 1024),
-                                                     16, voff[i], s * 128, 0, 0);
+        for (int i = 0; i < NI; i++) copy(cA, cB, s, lds + buf * C::SB + wave * NI * 1024, i);
     };
     float16_t acc[MI][NJ];
 #pragma unroll
@@ -588,31 +601,36 @@ __device__ __forceinline__ void gemmd_body(const GemmArgs &g, int m0, int n0, un
         for (int j = 0; j < NJ; j++) asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(fb[j]) : "v"(vb), "i"(j * 4096));
     };
     auto ready = [&](u4 (&fa)[MI], u4 (&fb)[NJ]) {
-        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        // the reads of later steps stay in flight (LDS reads return in order)
+        asm volatile("s_waitcnt lgkmcnt(%0)" ::"i"((C::D - 1) * (MI + NJ)) : "memory");
 #pragma unroll
         for (int i = 0; i < MI; i++) asm volatile("" : "+v"(fa[i]));
 #pragma unroll
         for (int j = 0; j < NJ; j++) asm volatile("" : "+v"(fb[j]));
     };
-    // Three stage buffers, four operand register sets (one per 16-k step of
-    // a stage).  Step st of stage s: wait for its operands (read during step
-    // st-1), then its MFMAs with step st+1's reads (into the set step st-3
-    // used) issued one after each MFMA.  At the last step every wave has its
-    // operands of the stage in registers: after one barrier (which also
-    // publishes the next stage's copies, waited for before it) the stage's
-    // buffer takes the copy of stage s+3, whose copy instructions go out one
-    // after each MFMA too, with the next stage's first reads.  Issued as a
+    // NS stage buffers, four operand register sets (one per 16-k step of a
+    // stage).  Step st of stage s: wait for its operands (read D steps
+    // before), then its MFMAs with the reads of step st + D and a quarter of
+    // the copies of stage s + NS - 1 issued one after each MFMA.  Issued as a
     // burst before the MFMAs, the reads and copies left the matrix pipe idle
     // for their issue time every step: interleaved, att.output at 4096 rows
-    // 70 -> 63 us, ffn.value 247 -> 232 us.
+    // 70 -> 63 us, ffn.value 247 -> 232 us.  The loop has no branch of its
+    // own: stages past the last are "copied" through resources of size 0
+    // (zeros into a free buffer, no memory traffic), and reads past the last
+    // fetch what is not used.  With the 18 scalar branches a stage that
+    // guarded them, 700 x 2560 x 2560 took 26.9 us where it takes 23.0 in
+    // the same 128x128 tiles, and 4096 x 7680 x 2560 155 where it takes 149.
     // step(): the MFMAs of operand set (ca, cb), with the LDS reads of set
-    // (na, nb) from stage offset boff (when rd) and the copies of stage ds
-    // into buffer db (when dm).
-    auto step = [&](const u4 (&ca)[MI], const u4 (&cb)[NJ], u4 (&na)[MI], u4 (&nb)[NJ], bool rd, uint32_t boff,
-                    int sn, bool dm, int ds, int db) {
+    // (na, nb), step sn, from stage offset boff and copies d0 .. d1 - 1 of
+    // stage ds into buffer db.
+    auto step = [&](const u4 (&ca)[MI], const u4 (&cb)[NJ], u4 (&na)[MI], u4 (&nb)[NJ], uint32_t boff, int sn, int ds, int db,
+                    int d0, int d1) {
         const uint32_t va = rowA + boff + xo[sn], vb = rowB + boff + xo[sn];
         unsigned char *dst = lds + db * C::SB + wave * NI * 1024;
-        int r = 0, d = 0;
+        const bool live = ds < nst;
+        const __amdgpu_buffer_rsrc_t cA = __builtin_amdgcn_make_buffer_rsrc((void *)g.a, (short)0, live ? sizeA : 0, 0x00020000);
+        const __amdgpu_buffer_rsrc_t cB = __builtin_amdgcn_make_buffer_rsrc((void *)g.b, (short)0, live ? sizeB : 0, 0x00020000);
+        int r = 0, d = d0;
 #pragma unroll
         for (int i = 0; i < MI; i++)
 #pragma unroll
@@ -620,62 +638,68 @@ __device__ __forceinline__ void gemmd_body(const GemmArgs &g, int m0, int n0, un
                 acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(half8_t, ca[i]),
                                                                  __builtin_bit_cast(half8_t, cb[j]), acc[i][j], 0, 0, 0);
                 __builtin_amdgcn_sched_barrier(0);
-                if (rd && r < MI + NJ) {
+                if (r < MI + NJ) {
                     if (r < MI) gd_read_piece(na[r], va, r);
                     else gd_read_piece(nb[r - MI], vb, r - MI);
                 }
                 r++;
                 __builtin_amdgcn_sched_barrier(0);
-                if (dm && d < NI)
-                    __builtin_amdgcn_raw_ptr_buffer_load_lds(d < nA ? rsA : rsB,
-                                                             (__attribute__((address_space(3))) void *)(dst + d * 1024), 16,
-                                                             voff[d], ds * 128, 0, 0);
+                if (d < d1) copy(cA, cB, ds, dst, d);
                 d++;
                 __builtin_amdgcn_sched_barrier(0);
             }
         // whatever did not fit between the MFMAs
 #pragma unroll
         for (; r < MI + NJ; r++) {
-            if (!rd) break;
             if (r < MI) gd_read_piece(na[r], va, r);
             else gd_read_piece(nb[r - MI], vb, r - MI);
         }
 #pragma unroll
-        for (; d < NI; d++) {
-            if (!dm) break;
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(d < nA ? rsA : rsB, (__attribute__((address_space(3))) void *)(dst + d * 1024),
-                                                     16, voff[d], ds * 128, 0, 0);
-        }
+        for (; d < d1; d++) copy(cA, cB, ds, dst, d);
         __builtin_amdgcn_sched_barrier(0);
     };
-    const int nst = g.k / 64;
-    issue(0, 0);
-    if (nst > 1) issue(1, 1);
-    if (nst > 2) issue(2, 2);
-    if (nst > 2) sk_wait_vm(2 * NI);
-    else if (nst > 1) sk_wait_vm(NI);
-    else sk_wait_vm(0);
+    // At step SBAR = 4 - D the next stage's operands are first read: its
+    // copies have landed, for every wave, after the wait and the barrier
+    // there, and every wave is past its last wait for operands of stage s - 1
+    // (D = 1: of stage s), whose buffer then takes the copies of stage
+    // s + NS - 1: at steps 0 .. 3 of stage s (D = 1) or steps 2, 3 of it and
+    // 0, 1 of stage s + 1 (D = 2; `late`).
+    constexpr int NS = C::NS, D = C::D;
+#pragma unroll
+    for (int i = 0; i < NS - 1; i++) issue(i, i);
+    static_assert((NS - 2) * NI < 63, "copies in flight fit the wait counter");
+    sk_wait_vm((NS - 2) * NI);
     __builtin_amdgcn_s_barrier();
     u4 fa[4][MI], fb[4][NJ];
-    read(fa[0], fb[0], 0, 0);
-    int buf = 0;
+#pragma unroll
+    for (int st = 0; st < D; st++) read(fa[st], fb[st], 0, st);
+    int buf = 0, pbuf = NS - 1, ppbuf = NS - 1;
     for (int s = 0; s < nst; s++) {
-        const int nbuf = buf == 2 ? 0 : buf + 1;
+        const int nbuf = buf == NS - 1 ? 0 : buf + 1;
 #pragma unroll
         for (int st = 0; st < 4; st++) {
             __builtin_amdgcn_sched_barrier(0);
             ready(fa[st], fb[st]);
-            if (st < 3) {
-                step(fa[st], fb[st], fa[st + 1], fb[st + 1], true, buf * C::SB, st + 1, false, 0, 0);
-            } else {
-                if (s + 2 < nst) sk_wait_vm(NI);
-                else sk_wait_vm(0);
+            constexpr int SBAR = 4 - D;
+            const bool late = D == 2 && st < SBAR;
+            const int part = D == 1 ? st : (st + 2) & 3, n = (st + D) & 3;
+            const int ds = late && s == 0 ? nst : s + NS - 1 - late, db = late ? ppbuf : pbuf;
+            if (st == SBAR) {
+                sk_wait_vm(D == 1 ? (NS - 3) * NI + NI * 3 / 4 : (NS - 3) * NI);  // stage s + 1 has landed
                 __builtin_amdgcn_s_barrier();
-                step(fa[3], fb[3], fa[0], fb[0], s + 1 < nst, nbuf * C::SB, 0, s + 3 < nst, s + 3, buf);
             }
+            step(fa[st], fb[st], fa[n], fb[n], (st >= SBAR ? nbuf : buf) * C::SB, n, ds, db, NI * part / 4,
+                 NI * (part + 1) / 4);
         }
+        ppbuf = pbuf;
+        pbuf = buf;
         buf = nbuf;
     }
+    // nothing in flight into registers or LDS past this point
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+#pragma unroll
+    for (int st = 0; st < D; st++) ready(fa[st], fb[st]);
+    sk_wait_vm(0);
     // 16-byte epilogue through LDS (the stage buffers are free once every
     // wave is past its last operand reads): each wave takes 32x36 floats
     const bool vec = g.n % 4 == 0 && g.ldc % 4 == 0;
@@ -817,11 +841,19 @@ static int gemm_check(const GemmArgs &g) {
     return 0;
 }
 
-// The DMA-tile form (fp16 weights, k % 64 == 0, offsets within 31 bits):
-// one of three tiles, whichever needs the fewest block rounds (one block per
-// CU) times tile area, weighted by the measured per-element cost of each form
-// (256x128 is the cheapest per element, 128x128 the dearest).
-enum GdKind { GD_NONE = 0, GD_256x160, GD_256x128, GD_128x128 };
+// The DMA-tile form (fp16 weights, k % 64 == 0, offsets within 31 bits): the
+// tile whose rounds over the chip (one block per CU) take the shortest.  A
+// full round of a tile takes `full` us at k = 2560, one that leaves most of
+// the chip idle `part` (the copies of an idle chip meet less traffic and its
+// clock is higher), in between in proportion; all scale with k alike.
+// Measured (us, tile 256x160 / 256x128 / 128x128 / 64x128 / 64x64):
+//    300 x  2560 x  2560:  35.3   29.5   21.5   17.3   11.5
+//    517 x  2560 x 10240:   117   99.4   71.4   49.5   64.4
+//    700 x  2560 x  2560:  35.6   30.9   22.4   18.3   19.8
+//   1500 x  2560 x  2560:  36.7   31.5   23.1   30.5   36.4
+//    517 x 10240 x  2560:  39.3   36.9   43.6   49.4   51.0
+//   4096 x  2560 x  2560:  54.4   79.5   78.5
+enum GdKind { GD_NONE = 0, GD_256x160, GD_256x128, GD_128x128, GD_64x128, GD_64x64 };
 
 static bool gd_fits(const GemmArgs &g) {
     return !g.b_i8 && g.k % 64 == 0 && (uint64_t)(g.m + 256) * g.lda * 2 < (1ull << 31) &&
@@ -829,20 +861,23 @@ static bool gd_fits(const GemmArgs &g) {
 }
 
 static int gd_tiles(const GemmArgs &g, int kind) {
-    const int bm = kind == GD_128x128 ? 128 : 256, bn = kind == GD_256x160 ? 160 : 128;
+    static const int bms[] = {0, 256, 256, 128, 64, 64}, bns[] = {0, 160, 128, 128, 128, 64};
+    const int bm = bms[kind], bn = bns[kind];
     return ((g.m + bm - 1) / bm) * ((g.n + bn - 1) / bn);
 }
 
 static GdKind gd_pick(const GemmArgs *gs, int n, int cus) {
     for (int i = 0; i < n; i++)
         if (!gd_fits(gs[i])) return GD_NONE;
-    static const double area[4] = {0, 256.0 * 160 * 1.0, 256.0 * 128 * 1.0, 128.0 * 128 * 1.2};
+    static const double part[] = {0, 34, 28.5, 19.5, 15.5, 10.5}, full[] = {0, 52, 42, 26, 16.5, 10.5};
     GdKind best = GD_NONE;
     double best_cost = 0;
-    for (int kind = GD_256x160; kind <= GD_128x128; kind++) {
+    for (int kind = GD_256x160; kind <= GD_64x64; kind++) {
         long tiles = 0;
         for (int i = 0; i < n; i++) tiles += gd_tiles(gs[i], kind);
-        const double cost = (double)((tiles + cus - 1) / cus) * area[kind];
+        const long rest = tiles % cus;
+        const double cost =
+            tiles / cus * full[kind] + (rest ? part[kind] + (full[kind] - part[kind]) * (double)rest / cus : 0.0);
         if (best == GD_NONE || cost < best_cost) best = (GdKind)kind, best_cost = cost;
     }
     return best;
@@ -868,7 +903,9 @@ int launch_gemm_multi(rsv_ctx *ctx, GemmJobs &jobs) {
         jobs.blk_start[jobs.n] = total;
         if (gk == GD_256x160) hipLaunchKernelGGL((k_gemmd_multi<4, 1, 2, 5>), dim3(total), dim3(256), 0, ctx->stream, jobs);
         else if (gk == GD_256x128) hipLaunchKernelGGL((k_gemmd_multi<2, 2, 4, 2>), dim3(total), dim3(256), 0, ctx->stream, jobs);
-        else hipLaunchKernelGGL((k_gemmd_multi<2, 2, 2, 2>), dim3(total), dim3(256), 0, ctx->stream, jobs);
+        else if (gk == GD_128x128) hipLaunchKernelGGL((k_gemmd_multi<2, 2, 2, 2>), dim3(total), dim3(256), 0, ctx->stream, jobs);
+        else if (gk == GD_64x128) hipLaunchKernelGGL((k_gemmd_multi<2, 2, 1, 2>), dim3(total), dim3(256), 0, ctx->stream, jobs);
+        else hipLaunchKernelGGL((k_gemmd_multi<2, 2, 1, 1>), dim3(total), dim3(256), 0, ctx->stream, jobs);
         RSV_HIP(hipGetLastError());
         return 0;
     }
@@ -893,7 +930,9 @@ int launch_gemm(rsv_ctx *ctx, const GemmArgs &g) {
         const dim3 gd_grid(gd_tiles(g, gk));
         if (gk == GD_256x160) hipLaunchKernelGGL((k_gemmd<4, 1, 2, 5>), gd_grid, dim3(256), 0, ctx->stream, g);
         else if (gk == GD_256x128) hipLaunchKernelGGL((k_gemmd<2, 2, 4, 2>), gd_grid, dim3(256), 0, ctx->stream, g);
-        else hipLaunchKernelGGL((k_gemmd<2, 2, 2, 2>), gd_grid, dim3(256), 0, ctx->stream, g);
+        else if (gk == GD_128x128) hipLaunchKernelGGL((k_gemmd<2, 2, 2, 2>), gd_grid, dim3(256), 0, ctx->stream, g);
+        else if (gk == GD_64x128) hipLaunchKernelGGL((k_gemmd<2, 2, 1, 2>), gd_grid, dim3(256), 0, ctx->stream, g);
+        else hipLaunchKernelGGL((k_gemmd<2, 2, 1, 1>), gd_grid, dim3(256), 0, ctx->stream, g);
         RSV_HIP(hipGetLastError());
         return 0;
     }

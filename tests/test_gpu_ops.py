@@ -973,6 +973,32 @@ def test_gemm_dma_tiles_equal_int8_loader(be, m, n, k):
     assert rel_err(g16.reshape(m, n), ref) < 1e-5
 
 
+@pytest.mark.parametrize("k", [64, 128, 192, 384, 2560])
+@pytest.mark.parametrize("m,n", [(1, 64), (63, 100), (65, 2562), (129, 5120), (191, 10240), (517, 2560), (1000, 2560)])
+def test_gemm_dma_tiles_agree_bit_for_bit(be, m, n, k):
+    """Few rows take the 64x64 and 64x128 tiles (then 128x128), many rows the
+    large ones: row r of an m-row product equals row r of the same product
+    over a chip-filling batch, bit for bit (one MFMA chain per element), for
+    every fill of the stage buffers (k / 64 from 1 up), n without the 16-byte
+    epilogue included; and float64 within the fp32 accumulation bound."""
+    rsv = _rsv()
+    rng = np.random.default_rng(m + 3 * n + k)
+    big = max(m, -(-256 * 256 * 160 // n) // 256 * 256)  # a 256x160 tile for every CU
+    big = min(big, 8192)
+    A = rng.standard_normal((big, k)).astype(np.float16)
+    W = (rng.standard_normal((n, k)) * k ** -0.5).astype(np.float16)
+    Wt = be.tensor(W.astype(np.float32), dtype=rsv.F16)
+    C = be.tensor(n=m * n)
+    be.call("rsv_gemm_ex", be.tensor(A[:m].astype(np.float32), dtype=rsv.F16), Wt, None, C, m, n, k, 0, NONE, NONE, NONE)
+    got = be.get(C, m * n).reshape(m, n)
+    Cb = be.tensor(n=big * n)
+    be.call("rsv_gemm_ex", be.tensor(A.astype(np.float32), dtype=rsv.F16), Wt, None, Cb, big, n, k, 0, NONE, NONE, NONE)
+    assert np.array_equal(got.view(np.uint32), be.get(Cb, big * n).reshape(big, n)[:m].view(np.uint32))
+    A64, W64 = A[:m].astype(np.float64), W.astype(np.float64)
+    bound = k * 2.0 ** -24 * (np.abs(A64) @ np.abs(W64).T)  # k additions of one rounding each
+    assert np.all(np.abs(got - A64 @ W64.T) <= bound)
+
+
 @pytest.mark.parametrize("m", [1030, 4096])
 def test_gemm_multi_fp16_jobs_equal_single_launches(be, m):
     """A job list of fp16 weights only (the prefill stage-1 list: r, k, v

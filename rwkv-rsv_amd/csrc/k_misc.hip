@@ -597,7 +597,8 @@ int launch_segmean(rsv_ctx *ctx, const float *x, float *out, const uint32_t *len
 namespace rsv {
 
 // ------------------------------------------------ packed prefill token mix
-// One block per token row, thread t owning the eight consecutive columns
+// One block per token row (two rows a block in launches that fill the chip so,
+// see k_seq_norm_mix), thread t owning the eight consecutive columns
 // 8t .. 8t+7 (c % 8 == 0, c <= 8192; blocks of c/8 threads rounded up to a
 // whole wave): 32-byte loads and 16-byte fp16 stores.  LN of the row and of
 // its predecessor (or the slot's token-shift state for the first row of a

@@ -971,9 +971,12 @@ __global__ __launch_bounds__(512) void k_wkv7_seq_cols(
 // and G by forward substitution, which keeps the error of the sequential order
 // where powers of A would not).  Then the state passes through the chunk as
 // U = P S'^T + G V, Y, S_end, each wave holding 16 state rows (rows are
-// independent).  Products, sums and everything kept stay fp32; the state's
-// error against 64 bits is that of the token-by-token scan (40 heads, 24
-// segments of 4096 tokens 8.5e-8 : 8.4e-8, 8 x 512 8.9e-8 : 8.4e-8).
+// independent).  Products, sums and everything kept stay fp32 (the products of
+// decays fp64); the state's error against 64 bits is below that of the
+// token-by-token scan: decays drawn per token 6.8e-8 : 7.2e-8 at every shape from
+// 1 x 40 to 24 segments of 4096.  Two things keep it there, sigma from 64 bits and
+// the order of the state's sums; with neither it was 8.1e-8 to 8.9e-8 (and 2 % of
+// the scan's time faster: 5 x 512 at 40 heads 99 -> 101 us).
 //   - S is held transposed in the MFMA accumulator layout: lane l, register
 //     (q, e) is S[row = l%16][column = 16q + 4(l/16) + e].  As the B operand of
 //     k-step (q, e) it is used in place: the four k of a step may be any four
@@ -1000,6 +1003,10 @@ struct WkvChunk {
 constexpr int kMmStep = 2;  // chunks of at most this many tokens are stepped token by token
 
 typedef float f4_t __attribute__((ext_vector_type(4)));
+// The row of token t in every array: the MFMA result layout then gives lane
+// group g, register e token 4e + g, so that the k-steps of a product over the
+// tokens take them in their order, oldest first.
+__device__ __forceinline__ constexpr int mm_row(int t) { return 4 * (t & 3) + (t >> 2); }
 __device__ __forceinline__ int mm64(int t, int c) { return t * 64 + (c ^ (t << 2)); }
 __device__ __forceinline__ int mm16(int t, int s) { return t * 16 + (s ^ (t >> 2 << 2)); }
 __device__ __forceinline__ f4_t mfma4(float a, float b, f4_t c) {
@@ -1017,6 +1024,23 @@ __device__ __forceinline__ float xsum_groups(float v) {
     v = __uint_as_float(p[0]) + __uint_as_float(p[1]);
     const auto q = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
     return __uint_as_float(q[0]) + __uint_as_float(q[1]);
+}
+// Two copies of v with their odd and even 16-lane groups (their halves)
+// swapped: the even and the odd group's (the lower and the upper half's) value
+// of the pair that the lane is in.
+__device__ __forceinline__ void swap16_d(double v, double &even, double &odd) {
+    const uint64_t b = __builtin_bit_cast(uint64_t, v);
+    const auto l = __builtin_amdgcn_permlane16_swap((uint32_t)b, (uint32_t)b, false, false);
+    const auto h = __builtin_amdgcn_permlane16_swap((uint32_t)(b >> 32), (uint32_t)(b >> 32), false, false);
+    even = __builtin_bit_cast(double, (uint64_t)h[0] << 32 | l[0]);
+    odd = __builtin_bit_cast(double, (uint64_t)h[1] << 32 | l[1]);
+}
+__device__ __forceinline__ void swap32_d(double v, double &low, double &high) {
+    const uint64_t b = __builtin_bit_cast(uint64_t, v);
+    const auto l = __builtin_amdgcn_permlane32_swap((uint32_t)b, (uint32_t)b, false, false);
+    const auto h = __builtin_amdgcn_permlane32_swap((uint32_t)(b >> 32), (uint32_t)(b >> 32), false, false);
+    low = __builtin_bit_cast(double, (uint64_t)h[0] << 32 | l[0]);
+    high = __builtin_bit_cast(double, (uint64_t)h[1] << 32 | l[1]);
 }
 // LDS made visible to the block; global loads and stores stay in flight
 __device__ __forceinline__ void lds_barrier() {
@@ -1060,7 +1084,7 @@ __device__ __forceinline__ void mm_plain(WkvChunk &c, const WkvTok &x, int lane,
     const int l16 = lane & 15, g = lane >> 4;
 #pragma unroll
     for (int i = 0; i < 4; i++) {
-        const int t = 4 * g + i, o = t * 64 + ((l16 ^ t) << 2), o2 = t * kMmLd + 4 * l16;
+        const int row = 4 * i + g, o = row * 64 + ((l16 ^ row) << 2), o2 = row * kMmLd + 4 * l16;
         const f4_t kh = x.k[i] * kkc * inv[i];
         *(f4_t *)&c.p[o2] = kh;
         *(f4_t *)&c.rt[o] = x.r[i];
@@ -1095,44 +1119,54 @@ __device__ __forceinline__ int mm_prepare(WkvChunk &c, WkvTok &x, uint32_t nt, i
     if (bonus && l16 < 4 && 4 * g + l16 < (int)nt)
         __builtin_nontemporal_store(l16 == 0 ? bs[0] : l16 == 1 ? bs[1] : l16 == 2 ? bs[2] : bs[3],
                                     bonus + (size_t)(4 * g + l16) * H);
-    // sigma of the lane's last token: the decays of the later groups' tokens
-    const f4_t pg = (x.w[0] * x.w[1]) * (x.w[2] * x.w[3]);
+    // sigma of the lane's last token: the decays of the later groups' tokens.
+    // Products of decays are formed in 64 bits (a multiplication costs what it does
+    // in 32) and rounded once: an error of sigma is one of a whole state column.
+    double sd[4];
     f4_t sg, rs;
 #pragma unroll
     for (int e = 0; e < 4; e++) {
-        const auto p16 = __builtin_amdgcn_permlane16_swap(__float_as_uint(pg[e]), __float_as_uint(pg[e]), false, false);
-        const float pair = __uint_as_float(p16[0]) * __uint_as_float(p16[1]);
-        const auto p32 = __builtin_amdgcn_permlane32_swap(__float_as_uint(pair), __float_as_uint(pair), false, false);
-        sg[e] = ((g & 1) ? 1.0f : __uint_as_float(p16[1])) * (g < 2 ? __uint_as_float(p32[1]) : 1.0f);
+        const double pg = ((double)x.w[0][e] * (double)x.w[1][e]) * ((double)x.w[2][e] * (double)x.w[3][e]);
+        double even, odd, low, high;
+        swap16_d(pg, even, odd);
+        swap32_d(even * odd, low, high);
+        sd[e] = ((g & 1) ? 1.0 : odd) * (g < 2 ? high : 1.0);
+        sg[e] = (float)sd[e];
         rs[e] = rcp_n(sg[e]);
     }
 #pragma unroll
     for (int i = 3; i >= 0; i--) {
-        const int t = 4 * g + i, o = t * 64 + ((l16 ^ t) << 2), o2 = t * kMmLd + 4 * l16;
+        const int row = 4 * i + g, o = row * 64 + ((l16 ^ row) << 2), o2 = row * kMmLd + 4 * l16;
         kk[i] *= inv[i];
         *(f4_t *)&c.bh[o2] = kk[i] * -x.a[i] * sg;
         *(f4_t *)&c.kh[o2] = km[i] * sg;
         *(f4_t *)&c.rt[o] = x.r[i] * rs;
-        sg *= x.w[i];
 #pragma unroll
-        for (int e = 0; e < 4; e++) rs[e] = rcp_n(sg[e]);
+        for (int e = 0; e < 4; e++) {
+            sd[e] *= (double)x.w[i][e];
+            sg[e] = (float)sd[e];
+            rs[e] = rcp_n(sg[e]);
+        }
         *(f4_t *)&c.p[o2] = kk[i] * rs;
     }
     if (g == 0) *(f4_t *)&c.dec[4 * l16] = sg;
-    f4_t ga = {0, 0, 0, 0}, gb = ga, gy = ga, gz = ga;
+    // A and Bm as four chains of 16 columns, added as a tree (they reach the state)
+    f4_t gaq[4], gbq[4], gy = {0, 0, 0, 0}, gz = gy;
 #pragma unroll
     for (int q = 0; q < 4; q++) {
+        gaq[q] = gbq[q] = (f4_t){0, 0, 0, 0};
         const int o = mm64(l16, 16 * q + 4 * g), o2 = l16 * kMmLd + 16 * q + 4 * g;
         const f4_t kt = *(const f4_t *)&c.p[o2], rt = *(const f4_t *)&c.rt[o], bh = *(const f4_t *)&c.bh[o2],
                    kh = *(const f4_t *)&c.kh[o2];
 #pragma unroll
         for (int e = 0; e < 4; e++) {
-            ga = mfma4(kt[e], bh[e], ga);
-            gb = mfma4(kt[e], kh[e], gb);
+            gaq[q] = mfma4(kt[e], bh[e], gaq[q]);
+            gbq[q] = mfma4(kt[e], kh[e], gbq[q]);
             gy = mfma4(rt[e], bh[e], gy);
             gz = mfma4(rt[e], kh[e], gz);
         }
     }
+    const f4_t ga = (gaq[0] + gaq[1]) + (gaq[2] + gaq[3]), gb = (gbq[0] + gbq[1]) + (gbq[2] + gbq[3]);
     // every scaled value meets a sum here, and values out of range leave one out
     // of range: 2^40, infinities and NaNs above it as bits
     // (and so must the decay over the chunk be, which the state is scaled by)
@@ -1154,14 +1188,15 @@ __device__ __forceinline__ int mm_prepare(WkvChunk &c, WkvTok &x, uint32_t nt, i
     fetch();
     __builtin_amdgcn_sched_barrier(0);
     if (step) return 1;
-    // A and Bm by row and column for the substitution
+    // A and Bm by token for the substitution
+    const int s16 = mm_row(l16);
 #pragma unroll
     for (int e = 0; e < 4; e++) {
-        const int t = 4 * g + e;
-        c.m[0][t * 16 + l16] = l16 < t ? ga[e] : 0.0f;
-        c.m[1][t * 16 + l16] = l16 < t ? gb[e] : 0.0f;
-        gy[e] = l16 <= t ? gy[e] : 0.0f;
-        gz[e] = l16 <= t ? gz[e] : 0.0f;
+        const int t = 4 * e + g;
+        c.m[0][t * 16 + s16] = s16 < t ? ga[e] : 0.0f;
+        c.m[1][t * 16 + s16] = s16 < t ? gb[e] : 0.0f;
+        gy[e] = s16 <= t ? gy[e] : 0.0f;
+        gz[e] = s16 <= t ? gz[e] : 0.0f;
     }
     // P and G row by row (lane = column; G's 16 columns in every group), the
     // next row of A read ahead
@@ -1169,7 +1204,7 @@ __device__ __forceinline__ int mm_prepare(WkvChunk &c, WkvTok &x, uint32_t nt, i
     f4_t at[4], an[4];
 #pragma unroll
     for (int t = 0; t < 16; t++) {
-        gk[t] = c.p[t * kMmLd + lane];
+        gk[t] = c.p[mm_row(t) * kMmLd + lane];
         gg[t] = c.m[1][t * 16 + l16];
     }
     at[0] = *(const f4_t *)&c.m[0][16];
@@ -1197,10 +1232,10 @@ __device__ __forceinline__ int mm_prepare(WkvChunk &c, WkvTok &x, uint32_t nt, i
     }
     // (the reads of m are done: LDS operations of a wave are in order)
 #pragma unroll
-    for (int t = 0; t < 16; t++) c.p[t * kMmLd + lane] = gk[t];
+    for (int t = 0; t < 16; t++) c.p[mm_row(t) * kMmLd + lane] = gk[t];
     if (g == 0) {
 #pragma unroll
-        for (int t = 0; t < 16; t++) c.m[0][mm16(t, l16)] = gg[t];
+        for (int t = 0; t < 16; t++) c.m[0][mm16(mm_row(t), s16)] = gg[t];
     }
 #pragma unroll
     for (int e = 0; e < 4; e++) {
@@ -1229,7 +1264,7 @@ __device__ __forceinline__ void mm_ops(WkvOps &o, const WkvChunk &c, int lane) {
 
 // The wave's 16 state rows through one prepared chunk, whose operands o were
 // read ahead; reads those of the next chunk n.  v: this lane's values of
-// tokens 4(l/16) + e, row l%16 (0 past the end); y as v.
+// tokens 4e + l/16, row l%16 (0 past the end); y as v.
 __device__ __forceinline__ void mm_consume(const WkvChunk &c, const WkvChunk &n, WkvOps &o, f4_t (&s)[4], const f4_t v,
                                            f4_t &y, int lane) {
     const int l16 = lane & 15, g = lane >> 4;
@@ -1245,58 +1280,56 @@ __device__ __forceinline__ void mm_consume(const WkvChunk &c, const WkvChunk &n,
             bh[e][q] = c.bh[(4 * g + e) * kMmLd + 16 * q + l16];
         }
     const f4_t my = *(const f4_t *)&c.m[1][mm16(l16, 4 * g)];
-    // one chain of 16 columns per q, added as a tree
-    f4_t u[4], z[4];
+    // U and rt S'^T as one chain of 16 columns per q, added as a tree
+    f4_t u[4], z[4], ub[4];
 #pragma unroll
     for (int q = 0; q < 4; q++) {
         s[q] *= o.dec[q];
-        u[q] = z[q] = (f4_t){0, 0, 0, 0};
+        u[q] = z[q] = ub[q] = (f4_t){0, 0, 0, 0};
     }
     f4_t ug = {0, 0, 0, 0}, yz = ug;
 #pragma unroll
     for (int e = 0; e < 4; e++) {
         ug = mfma4(o.mg[e], v[e], ug);
-        yz = mfma4(o.mz[e], v[e], yz);
+#pragma unroll
+        for (int q = 0; q < 4; q++) u[q] = mfma4(o.p[q][e], s[q][e], u[q]);
     }
+    const f4_t us = ((u[0] + u[1]) + (u[2] + u[3])) + ug;
 #pragma unroll
-    for (int e = 0; e < 4; e++)
+    for (int e = 0; e < 4; e++) {
+        yz = mfma4(o.mz[e], v[e], yz);
 #pragma unroll
-        for (int q = 0; q < 4; q++) {
-            u[q] = mfma4(o.p[q][e], s[q][e], u[q]);
-            z[q] = mfma4(o.rt[q][e], s[q][e], z[q]);
-        }
+        for (int q = 0; q < 4; q++) z[q] = mfma4(o.rt[q][e], s[q][e], z[q]);
+    }
 #pragma unroll
     for (int i = 0; i < 40; i++) {
         __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // a product
         __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);  // an LDS read
     }
     __builtin_amdgcn_sched_barrier(0);
-    // V^T kh in sums of its own: one rounding at the state's size instead of 16
-    // (with the chain begun at S' the state's error was 1.2e-7 against 8e-8)
-    f4_t vk[4];
-#pragma unroll
-    for (int q = 0; q < 4; q++) vk[q] = (f4_t){0, 0, 0, 0};
+    mm_ops(o, n, lane);
+    // U^T bh in sums of its own, then V^T kh onto S' + U^T bh, oldest token
+    // first: the sums reach the state's size only with the last tokens, as they do
+    // token by token (the error of the state: see the top)
 #pragma unroll
     for (int e = 0; e < 4; e++)
 #pragma unroll
-        for (int q = 0; q < 4; q++) vk[q] = mfma4(kh[e][q], v[e], vk[q]);
-    const f4_t us = ((u[0] + u[1]) + (u[2] + u[3])) + ug;
-    __builtin_amdgcn_sched_barrier(0);
-    mm_ops(o, n, lane);
+        for (int q = 0; q < 4; q++) ub[q] = mfma4(bh[e][q], us[e], ub[q]);
 #pragma unroll
-    for (int e = 0; e < 4; e++) {
-#pragma unroll
-        for (int q = 0; q < 4; q++) s[q] = mfma4(bh[e][q], us[e], s[q]);
-        yz = mfma4(my[e], us[e], yz);
+    for (int q = 0; q < 4; q++) {
+        yz = mfma4(my[q], us[q], yz);
+        s[q] += ub[q];
     }
 #pragma unroll
-    for (int i = 0; i < 20; i++) {
+    for (int e = 0; e < 4; e++)
+#pragma unroll
+        for (int q = 0; q < 4; q++) s[q] = mfma4(kh[e][q], v[e], s[q]);
+#pragma unroll
+    for (int i = 0; i < 36; i++) {
         __builtin_amdgcn_sched_group_barrier(0x008, 1, 1);
         __builtin_amdgcn_sched_group_barrier(0x100, 1, 1);
     }
     __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-    for (int q = 0; q < 4; q++) s[q] += vk[q];
     y = ((z[0] + z[1]) + (z[2] + z[3])) + yz;
 }
 
@@ -1306,20 +1339,21 @@ __device__ __forceinline__ void mm_step(const WkvChunk &c, f4_t (&s)[4], const f
     asm volatile("" : "+v"(lane));
     const int l16 = lane & 15, g = lane >> 4;
     for (uint32_t t = 0; t < nt; t++) {
-        const float vt = __shfl((t & 3) == 0 ? v[0] : (t & 3) == 1 ? v[1] : (t & 3) == 2 ? v[2] : v[3], 16 * (int)(t >> 2) + l16);
+        const int row = mm_row((int)t);
+        const float vt = __shfl(t < 4 ? v[0] : t < 8 ? v[1] : t < 12 ? v[2] : v[3], 16 * (int)(t & 3) + l16);
         float sa = 0.0f, yt = 0.0f;
 #pragma unroll
         for (int q = 0; q < 4; q++) {
-            const f4_t kh = *(const f4_t *)&c.p[t * kMmLd + 16 * q + 4 * g];
+            const f4_t kh = *(const f4_t *)&c.p[row * kMmLd + 16 * q + 4 * g];
 #pragma unroll
             for (int e = 0; e < 4; e++) sa = fmaf(s[q][e], kh[e], sa);
         }
         sa = xsum_groups(sa);
 #pragma unroll
         for (int q = 0; q < 4; q++) {
-            const int o = mm64(t, 16 * q + 4 * g);
+            const int o = mm64(row, 16 * q + 4 * g);
             const f4_t wt = *(const f4_t *)(w + t * C + 16 * q + 4 * g);
-            const f4_t b = *(const f4_t *)&c.bh[t * kMmLd + 16 * q + 4 * g], km = *(const f4_t *)&c.kh[t * kMmLd + 16 * q + 4 * g],
+            const f4_t b = *(const f4_t *)&c.bh[row * kMmLd + 16 * q + 4 * g], km = *(const f4_t *)&c.kh[row * kMmLd + 16 * q + 4 * g],
                        rt = *(const f4_t *)&c.rt[o];
 #pragma unroll
             for (int e = 0; e < 4; e++) {
@@ -1329,7 +1363,7 @@ __device__ __forceinline__ void mm_step(const WkvChunk &c, f4_t (&s)[4], const f
         }
         yt = xsum_groups(yt);
 #pragma unroll
-        for (int e = 0; e < 4; e++) y[e] = (int)t == 4 * g + e ? yt : y[e];
+        for (int e = 0; e < 4; e++) y[e] = (int)t == 4 * e + g ? yt : y[e];
     }
 }
 
@@ -1387,7 +1421,7 @@ __global__ __launch_bounds__(64 * (NC + NP), (NC + NP) / 4) void k_wkv7_seq_mm(
         for (int i = 0; i < NP; i++) {
             const __amdgpu_buffer_rsrc_t bv = mm_rsrc(v + col + (size_t)(tb + 16 * i) * C, C, ntok(tb + 16 * i));
 #pragma unroll
-            for (int e = 0; e < 4; e++) z[i][e] = mm_ld(bv, ((4 * g + e) * (int)C + 16 * pw + l16) * 4);
+            for (int e = 0; e < 4; e++) z[i][e] = mm_ld(bv, ((4 * e + g) * (int)C + 16 * pw + l16) * 4);
         }
     };
     f4_t s[4];
@@ -1431,11 +1465,11 @@ __global__ __launch_bounds__(64 * (NC + NP), (NC + NP) / 4) void k_wkv7_seq_mm(
             if (poison) {
                 int first = 16;  // the row's first such token
 #pragma unroll
-                for (int e = 3; e >= 0; e--) first = fabsf(vraw[e]) <= 3.4028235e38f ? first : 4 * g + e;
+                for (int e = 3; e >= 0; e--) first = fabsf(vraw[e]) <= 3.4028235e38f ? first : 4 * e + g;
                 first = min(first, __shfl_xor(first, 16));
                 first = min(first, __shfl_xor(first, 32));
 #pragma unroll
-                for (int e = 0; e < 4; e++) y[e] = 4 * g + e >= first ? __builtin_nanf("") : y[e];
+                for (int e = 0; e < 4; e++) y[e] = 4 * e + g >= first ? __builtin_nanf("") : y[e];
 #pragma unroll
                 for (int q = 0; q < 4; q++)
 #pragma unroll
@@ -1450,7 +1484,7 @@ __global__ __launch_bounds__(64 * (NC + NP), (NC + NP) / 4) void k_wkv7_seq_mm(
             const __amdgpu_buffer_rsrc_t by = mm_rsrc(y_out + col + (size_t)tb * C, C, nt);
 #pragma unroll
             for (int e = 0; e < 4; e++)
-                __builtin_amdgcn_raw_buffer_store_b32(__float_as_int(y[e]), by, ((4 * g + e) * (int)C + 16 * pw + l16) * 4, 0, kNt);
+                __builtin_amdgcn_raw_buffer_store_b32(__float_as_int(y[e]), by, ((4 * e + g) * (int)C + 16 * pw + l16) * 4, 0, kNt);
         }
     }
 #pragma unroll

@@ -401,6 +401,43 @@ def test_seq_norm_mix_rows(be, T, c, nout):
 
 
 @pytest.mark.parametrize("form", ["4", "1"])
+@pytest.mark.parametrize("decays", ["token", "channel"])
+def test_wkv7_seq_chunked_state_error_against_64_bits(be, decays, form, monkeypatch):
+    """The chunked scan may not lose precision: its state is no further from
+    64 bits (2-norm) than the token-by-token form's, with decays drawn
+    for each token, where the last few tokens' roundings count, and decays of the
+    channel, where those of hundreds of tokens add up."""
+    rsv = _rsv()
+    H, lens = 4, [40, 200, 460]
+    C, T, n = H * 64, sum(lens), len(lens)
+    rng = np.random.default_rng(11)
+    r, v, k, _, a, _, kk, ka, rk, gam, bet = _wkv_inputs(rng, T, H)
+    x = rng.standard_normal((T, C)) * 2 - 1.5 if decays == "token" else rng.standard_normal(C) * 2 - 1.5 + rng.standard_normal((T, C)) * 0.5
+    w = np.exp(-0.6065 / (1 + np.exp(-x))).astype(np.float32)
+    S = (rng.standard_normal((n, H, 64, 64)) * 0.1).astype(np.float32)
+    starts = np.concatenate([[0], np.cumsum(lens)[:-1]])
+    k64, v64, w64, a64 = (z.astype(np.float64).reshape(T, H, 64) for z in (k, v, w, a))
+    kh = k64 * kk.reshape(H, 64)
+    kh /= np.sqrt((kh * kh).sum(2, keepdims=True))
+    km = k64 + ka.astype(np.float64).reshape(H, 64) * (k64 * a64 - k64)
+    want = S.astype(np.float64)
+    for i, (t0, m) in enumerate(zip(starts, lens)):
+        for t in range(t0, t0 + m):
+            sa = np.matmul(want[i], kh[t][:, :, None])
+            want[i] = want[i] * w64[t][:, None, :] - sa * (kh[t] * a64[t])[:, None, :] + v64[t][:, :, None] * km[t][:, None, :]
+    st, ln, sl = (be.tensor(np.asarray(z, np.uint32), dtype=rsv.U32) for z in (starts, lens, range(n)))
+    common = [be.tensor(z) for z in (r, w, k, v, a, kk, ka, rk, gam, bet)]
+    err = []
+    for which in ("0", form):
+        monkeypatch.setenv("RSV_SCAN_G", which)
+        s2, gt, yw, bw = be.tensor(S), be.tensor(a), be.tensor(n=T * C), be.tensor(n=T * H)
+        yg = be.tensor(n=T * C, dtype=rsv.F16)
+        be.call("rsv_wkv7_seq_ragged_gate", s2, *common, gt, yw, bw, yg, st, ln, sl, n, T, H, 64, 64e-5)
+        err.append(np.linalg.norm(be.get(s2, S.size) - want.reshape(-1)) / np.linalg.norm(want))
+    assert err[1] <= err[0], err
+
+
+@pytest.mark.parametrize("form", ["4", "1"])
 @pytest.mark.parametrize("kind", ["model", "strong", "big", "nan_k", "inf_v"])
 def test_wkv7_seq_chunked_matches_token_by_token(be, kind, form, monkeypatch):
     """The chunked scan (whole heads and quarters per block) against the

@@ -1112,9 +1112,10 @@ __device__ __forceinline__ int mm_prepare(WkvChunk &c, WkvTok &x, uint32_t nt, i
         const f4_t q = kk[i] * kk[i], z = x.r[i] * km[i] * rk;
         const float ss = row16_sum((q[0] + q[1]) + (q[2] + q[3]));
         bs[i] = row16_sum((z[0] + z[1]) + (z[2] + z[3]));
-        // 1 / max(|kk|, eps): reciprocal root and one Newton step
+        // 1 / max(|kk|, eps): reciprocal root and one Newton step (not for a sum that
+        // overflowed: its 0 stands, as 1 / sqrt(inf) does token by token)
         const float y = __builtin_amdgcn_rsqf(ss);
-        inv[i] = ss < eps * eps ? 1.0f / eps : fmaf(0.5f * y, fmaf(-ss * y, y, 1.0f), y);
+        inv[i] = ss < eps * eps ? 1.0f / eps : y == 0.0f ? 0.0f : fmaf(0.5f * y, fmaf(-ss * y, y, 1.0f), y);
     }
     if (bonus && l16 < 4 && 4 * g + l16 < (int)nt)
         __builtin_nontemporal_store(l16 == 0 ? bs[0] : l16 == 1 ? bs[1] : l16 == 2 ? bs[2] : bs[3],

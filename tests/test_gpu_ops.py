@@ -438,13 +438,14 @@ def test_wkv7_seq_chunked_state_error_against_64_bits(be, decays, form, monkeypa
 
 
 @pytest.mark.parametrize("form", ["4", "1"])
-@pytest.mark.parametrize("kind", ["model", "strong", "big", "nan_k", "inf_v"])
+@pytest.mark.parametrize("kind", ["model", "strong", "big", "over", "nan_k", "inf_v"])
 def test_wkv7_seq_chunked_matches_token_by_token(be, kind, form, monkeypatch):
     """The chunked scan (whole heads and quarters per block) against the
     token-by-token form, at segment lengths around its chunks of 16 and its
     supersteps of 48 and 64 tokens: decays of the model, decays down to 0 and
-    keys of 1e13 (both leave its range and are stepped token by token), and
-    inputs that are not finite, which must reach the same tokens and rows.
+    keys of 1e13 (both leave its range and are stepped token by token), finite
+    keys whose sum of squares overflows (k^ = 0, no NaN), and inputs that are
+    not finite, which must reach the same tokens and rows.
     The two sum in another order: a few hundred roundings of 2^-24 (state), a
     16-bit output (yg)."""
     rsv = _rsv()
@@ -459,6 +460,9 @@ def test_wkv7_seq_chunked_matches_token_by_token(be, kind, form, monkeypatch):
         w[rng.random((T, C)) < 0.02] = 0.0
     elif kind == "big":
         k, rk = k * np.float32(1e13), rk * 0  # (no bonus: it would leave fp16's range)
+    elif kind == "over":
+        k[T - 60, 64:128] *= np.float32(1e20)
+        rk = rk * 0
     elif kind == "nan_k":
         k[T - 60, 70] = np.nan  # head 1 of the last segment
     elif kind == "inf_v":

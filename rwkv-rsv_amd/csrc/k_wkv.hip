@@ -988,17 +988,19 @@ __global__ __launch_bounds__(512) void k_wkv7_seq_cols(
 //     p ^ (t/4).  All reads are free of bank conflicts.
 //   - A chunk whose Gram products pass 2^40 or are not finite (strong decays, or
 //     inputs not finite), where 0 * inf would reach the chunk's earlier tokens, is
-//     stepped token by token by the same waves, and so is one of few tokens (a
-//     decode row packed among prompts).
+//     stepped token by token, from memory, by the waves that hold the state, and so
+//     is one of few tokens (a decode row packed among prompts), one whose v is not
+//     finite and any while the state is not: what an infinity leaves behind is
+//     the token-by-token form's.
 constexpr int kNt = 2;  // cache policy of a buffer store: non-temporal
 constexpr int kMmLd = 68;
 struct WkvChunk {
-    float p[16 * kMmLd];    // P            (token by token: k^)
-    float rt[16 * 64];      // rt           (r)
-    float bh[16 * kMmLd];   // bh           (-k^ a)
-    float kh[16 * kMmLd];   // kh           (k_mod); [64], between rows: whether to step token by token
-    float m[3][16 * 16];    // G, Ay, By
-    float dec[64];          // sigma_{-1}
+    float p[16 * kMmLd];   // P
+    float rt[16 * 64];     // rt
+    float bh[16 * kMmLd];  // bh
+    float kh[16 * kMmLd];  // kh; [64], between rows: whether to step token by token (the rest is then not read)
+    float m[3][16 * 16];   // G, Ay, By
+    float dec[64];         // sigma_{-1}
 };
 constexpr int kMmStep = 2;  // chunks of at most this many tokens are stepped token by token
 
@@ -1079,26 +1081,12 @@ __device__ __forceinline__ void mm_load(WkvTok &x, const float *__restrict__ k, 
     }
 }
 
-// The token-by-token vectors of a chunk: k^ (kk scaled by inv), r, -k^ a, k_mod.
-__device__ __forceinline__ void mm_plain(WkvChunk &c, const WkvTok &x, int lane, f4_t kkc, f4_t ka, const float (&inv)[4]) {
-    const int l16 = lane & 15, g = lane >> 4;
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
-        const int row = 4 * i + g, o = row * 64 + ((l16 ^ row) << 2), o2 = row * kMmLd + 4 * l16;
-        const f4_t kh = x.k[i] * kkc * inv[i];
-        *(f4_t *)&c.p[o2] = kh;
-        *(f4_t *)&c.rt[o] = x.r[i];
-        *(f4_t *)&c.bh[o2] = kh * -x.a[i];
-        *(f4_t *)&c.kh[o2] = x.k[i] + ka * (x.k[i] * x.a[i] - x.k[i]);
-    }
-}
-
 // One wave prepares one chunk of nt tokens (1..16) in LDS; returns whether it
-// is to be stepped token by token.  load(y) reads the chunk again (the rare
-// token-by-token case); fetch() reads the wave's next chunk into x.
-template <class L, class F>
+// is to be stepped token by token instead.  fetch() reads the wave's next chunk
+// into x.
+template <class F>
 __device__ __forceinline__ int mm_prepare(WkvChunk &c, WkvTok &x, uint32_t nt, int lane, f4_t kkc, f4_t ka, f4_t rk,
-                                          float eps, float *__restrict__ bonus, int H, L load, F fetch) {
+                                          float eps, float *__restrict__ bonus, int H, F fetch) {
     asm volatile("" : "+v"(lane));  // LDS addresses formed here, not kept in registers around the chunk loop
     const int l16 = lane & 15, g = lane >> 4;
     f4_t kk[4], km[4];
@@ -1120,6 +1108,10 @@ __device__ __forceinline__ int mm_prepare(WkvChunk &c, WkvTok &x, uint32_t nt, i
     if (bonus && l16 < 4 && 4 * g + l16 < (int)nt)
         __builtin_nontemporal_store(l16 == 0 ? bs[0] : l16 == 1 ? bs[1] : l16 == 2 ? bs[2] : bs[3],
                                     bonus + (size_t)(4 * g + l16) * H);
+    if (nt <= (uint32_t)kMmStep) {
+        fetch();
+        return 1;
+    }
     // sigma of the lane's last token: the decays of the later groups' tokens.
     // Products of decays are formed in 64 bits (a multiplication costs what it does
     // in 32) and rounded once: an error of sigma is one of a whole state column.
@@ -1179,12 +1171,7 @@ __device__ __forceinline__ int mm_prepare(WkvChunk &c, WkvTok &x, uint32_t nt, i
     for (int e = 0; e < 4; e++)
         mag = max(max(max(mag, __float_as_uint(ga[e]) & 0x7FFFFFFFu), max(__float_as_uint(gb[e]) & 0x7FFFFFFFu, __float_as_uint(gy[e]) & 0x7FFFFFFFu)),
                   __float_as_uint(gz[e]) & 0x7FFFFFFFu);
-    const bool step = __ballot(mag >= 0x53800000u) != 0 || nt <= (uint32_t)kMmStep;
-    if (step) {
-        WkvTok y;
-        load(y);
-        mm_plain(c, y, lane, kkc, ka, inv);
-    }
+    const bool step = __ballot(mag >= 0x53800000u) != 0;
     __builtin_amdgcn_sched_barrier(0);
     fetch();
     __builtin_amdgcn_sched_barrier(0);
@@ -1334,28 +1321,39 @@ __device__ __forceinline__ void mm_consume(const WkvChunk &c, const WkvChunk &n,
     y = ((z[0] + z[1]) + (z[2] + z[3])) + yz;
 }
 
-// The same, token by token, on the plain vectors (see WkvChunk).
-__device__ __forceinline__ void mm_step(const WkvChunk &c, f4_t (&s)[4], const f4_t v, f4_t &y, int lane,
-                                        const float *__restrict__ w, size_t C, uint32_t nt) {
+// The same, token by token, from the inputs (offset to the chunk and the head).
+__device__ __forceinline__ void mm_step(f4_t (&s)[4], const f4_t v, f4_t &y, int lane, const float *__restrict__ k,
+                                        const float *__restrict__ a, const float *__restrict__ w,
+                                        const float *__restrict__ r, const float *__restrict__ kkc,
+                                        const float *__restrict__ ka, float eps, size_t C, uint32_t nt) {
     asm volatile("" : "+v"(lane));
     const int l16 = lane & 15, g = lane >> 4;
     for (uint32_t t = 0; t < nt; t++) {
-        const int row = mm_row((int)t);
         const float vt = __shfl(t < 4 ? v[0] : t < 8 ? v[1] : t < 12 ? v[2] : v[3], 16 * (int)(t & 3) + l16);
-        float sa = 0.0f, yt = 0.0f;
+        const size_t o = t * C + 4 * g;
+        f4_t kh[4];
+        float ss = 0.0f, sa = 0.0f, yt = 0.0f;
 #pragma unroll
         for (int q = 0; q < 4; q++) {
-            const f4_t kh = *(const f4_t *)&c.p[row * kMmLd + 16 * q + 4 * g];
+            kh[q] = *(const f4_t *)(k + o + 16 * q) * *(const f4_t *)(kkc + 16 * q + 4 * g);
 #pragma unroll
-            for (int e = 0; e < 4; e++) sa = fmaf(s[q][e], kh[e], sa);
+            for (int e = 0; e < 4; e++) ss = fmaf(kh[q][e], kh[q][e], ss);
+        }
+        float nrm = sqrtf(xsum_groups(ss));
+        nrm = nrm < eps ? eps : nrm;
+        const float inv = 1.0f / nrm;
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            kh[q] *= inv;
+#pragma unroll
+            for (int e = 0; e < 4; e++) sa = fmaf(s[q][e], kh[q][e], sa);
         }
         sa = xsum_groups(sa);
 #pragma unroll
         for (int q = 0; q < 4; q++) {
-            const int o = mm64(row, 16 * q + 4 * g);
-            const f4_t wt = *(const f4_t *)(w + t * C + 16 * q + 4 * g);
-            const f4_t b = *(const f4_t *)&c.bh[row * kMmLd + 16 * q + 4 * g], km = *(const f4_t *)&c.kh[row * kMmLd + 16 * q + 4 * g],
-                       rt = *(const f4_t *)&c.rt[o];
+            const f4_t kt = *(const f4_t *)(k + o + 16 * q), at = *(const f4_t *)(a + o + 16 * q), wt = *(const f4_t *)(w + o + 16 * q),
+                       rt = *(const f4_t *)(r + o + 16 * q);
+            const f4_t b = kh[q] * -at, km = kt + *(const f4_t *)(ka + 16 * q + 4 * g) * (kt * at - kt);
 #pragma unroll
             for (int e = 0; e < 4; e++) {
                 s[q][e] = s[q][e] * wt[e] + sa * b[e] + vt * km[e];
@@ -1368,6 +1366,16 @@ __device__ __forceinline__ void mm_step(const WkvChunk &c, f4_t (&s)[4], const f
     }
 }
 
+// Whether any of the wave's state elements is not finite.
+__device__ __forceinline__ bool mm_wild(const f4_t (&s)[4]) {
+    bool fine = true;
+#pragma unroll
+    for (int q = 0; q < 4; q++)
+#pragma unroll
+        for (int e = 0; e < 4; e++) fine = fine && fabsf(s[q][e]) <= 3.4028235e38f;
+    return __ballot(!fine) != 0;
+}
+
 // One block per (head, segment, 4/NC-th of its rows): waves NC.. prepare the
 // next NP chunks, one each, into one set while waves 0..NC-1 pass the state's
 // rows, 16 each, through the NP chunks of the other.
@@ -1375,8 +1383,10 @@ __device__ __forceinline__ void mm_step(const WkvChunk &c, f4_t (&s)[4], const f
 //   <1, 3>: a quarter of the rows per block, for launches that leave CUs idle.
 //     fp32 MFMA holds its SIMD's VALU for half of its 32 cycles, so a preparing
 //     wave beside a passing one slows both; here each has a SIMD of its own.
+// (Bounds of 512 threads for both: with one wave per SIMD allowed for <1, 3> the
+// compiler keeps the sums in AGPRs and moves them through VGPRs for each addition.)
 template <int NC, int NP>
-__global__ __launch_bounds__(64 * (NC + NP), (NC + NP) / 4) void k_wkv7_seq_mm(
+__global__ __launch_bounds__(512, 2) void k_wkv7_seq_mm(
     float *__restrict__ S, const float *__restrict__ r, const float *__restrict__ w, const float *__restrict__ k,
     const float *__restrict__ v, const float *__restrict__ a, const float *__restrict__ kkc,
     const float *__restrict__ ka, const float *__restrict__ rk, float *__restrict__ y_out,
@@ -1407,7 +1417,7 @@ __global__ __launch_bounds__(64 * (NC + NP), (NC + NP) / 4) void k_wkv7_seq_mm(
                 float *bonus = blockIdx.z == 0 ? bonus_out + (size_t)(t0 + tb) * H + h : nullptr;
                 WkvChunk &c = chunk[sup & 1][pw];
                 const int st = mm_prepare(c, x, nt, lane, kkc_j, ka_j, rk_j, eps, bonus, H,
-                                          [&](WkvTok &y) { load(y, tb); }, [&] { load(x, tb + kSup); });
+                                          [&] { load(x, tb + kSup); });
                 if (lane == 0) c.kh[64] = __int_as_float(st);
             }
             lds_barrier();
@@ -1428,14 +1438,15 @@ __global__ __launch_bounds__(64 * (NC + NP), (NC + NP) / 4) void k_wkv7_seq_mm(
     f4_t s[4];
 #pragma unroll
     for (int q = 0; q < 4; q++) s[q] = *(const f4_t *)(Srow + 16 * q + 4 * g);
+    bool wild = mm_wild(s);
     f4_t vn[NP];
     vload(vn, 0);
     for (uint32_t sup = 0; sup < nsup; sup++) {
         const int set = sup & 1;
         lds_barrier();
-        WkvOps o;
+        WkvOps ops;
         const int stepped = __float_as_int(chunk[set][lane < NP ? lane : 0].kh[64]);
-        mm_ops(o, chunk[set][0], lane);
+        mm_ops(ops, chunk[set][0], lane);
         f4_t vs[NP];
 #pragma unroll
         for (int i = 0; i < NP; i++) vs[i] = vn[i];
@@ -1447,34 +1458,15 @@ __global__ __launch_bounds__(64 * (NC + NP), (NC + NP) / 4) void k_wkv7_seq_mm(
             f4_t vc = vs[0], y;
 #pragma unroll
             for (int j = 0; j < NP - 1; j++) vs[j] = vs[j + 1];
-            // a value of v that is not finite stays out of the products (0 * inf
-            // would reach earlier tokens) and is put on the row's later tokens
-            // and state below
-            const bool poison = __ballot(!((fabsf(vc[0]) + fabsf(vc[1])) + (fabsf(vc[2]) + fabsf(vc[3])) <= 3.4028235e38f)) != 0;
-            const f4_t vraw = vc;
-            if (poison) {
-#pragma unroll
-                for (int e = 0; e < 4; e++) vc[e] = fabsf(vc[e]) <= 3.4028235e38f ? vc[e] : 0.0f;
-            }
             const WkvChunk &next = chunk[set][i < NP - 1 ? i + 1 : i];
-            if (__builtin_amdgcn_readlane(stepped, i)) {
-                mm_step(chunk[set][i], s, vc, y, lane, w + col + (size_t)tb * C, C, nt);
-                mm_ops(o, next, lane);
+            const bool vfine = (fabsf(vc[0]) + fabsf(vc[1])) + (fabsf(vc[2]) + fabsf(vc[3])) <= 3.4028235e38f;
+            if (__builtin_amdgcn_readlane(stepped, i) || wild || __ballot(!vfine) != 0) {
+                const size_t o = col + (size_t)tb * C;
+                mm_step(s, vc, y, lane, k + o, a + o, w + o, r + o, kkc + h * 64, ka + h * 64, eps, C, nt);
+                wild = mm_wild(s);
+                mm_ops(ops, next, lane);
             } else {
-                mm_consume(chunk[set][i], next, o, s, vc, y, lane);
-            }
-            if (poison) {
-                int first = 16;  // the row's first such token
-#pragma unroll
-                for (int e = 3; e >= 0; e--) first = fabsf(vraw[e]) <= 3.4028235e38f ? first : 4 * e + g;
-                first = min(first, __shfl_xor(first, 16));
-                first = min(first, __shfl_xor(first, 32));
-#pragma unroll
-                for (int e = 0; e < 4; e++) y[e] = 4 * e + g >= first ? __builtin_nanf("") : y[e];
-#pragma unroll
-                for (int q = 0; q < 4; q++)
-#pragma unroll
-                    for (int e = 0; e < 4; e++) s[q][e] = first < 16 ? __builtin_nanf("") : s[q][e];
+                mm_consume(chunk[set][i], next, ops, s, vc, y, lane);
             }
             // wait for the next superstep's v here: after these stores the wait
             // would be for them too

@@ -438,14 +438,15 @@ def test_wkv7_seq_chunked_state_error_against_64_bits(be, decays, form, monkeypa
 
 
 @pytest.mark.parametrize("form", ["4", "1"])
-@pytest.mark.parametrize("kind", ["model", "strong", "big", "over", "nan_k", "inf_v"])
+@pytest.mark.parametrize("kind", ["model", "strong", "big", "over", "nan_k", "inf_v", "inf_v_last", "inf_s"])
 def test_wkv7_seq_chunked_matches_token_by_token(be, kind, form, monkeypatch):
     """The chunked scan (whole heads and quarters per block) against the
     token-by-token form, at segment lengths around its chunks of 16 and its
     supersteps of 48 and 64 tokens: decays of the model, decays down to 0 and
     keys of 1e13 (both leave its range and are stepped token by token), finite
-    keys whose sum of squares overflows (k^ = 0, no NaN), and inputs that are
-    not finite, which must reach the same tokens and rows.
+    keys whose sum of squares overflows (k^ = 0, no NaN), and inputs or a state
+    that are not finite, which must reach the same tokens and rows and leave the
+    same infinities and NaNs.
     The two sum in another order: a few hundred roundings of 2^-24 (state), a
     16-bit output (yg)."""
     rsv = _rsv()
@@ -467,9 +468,13 @@ def test_wkv7_seq_chunked_matches_token_by_token(be, kind, form, monkeypatch):
         k[T - 60, 70] = np.nan  # head 1 of the last segment
     elif kind == "inf_v":
         v[T - 60, 130] = np.inf  # one state row of head 2
+    elif kind == "inf_v_last":
+        v[np.cumsum(lens)[3:] - 1, 130] = -np.inf  # at a segment's end, where the state's infinities are left
     g = rng.random((T, C)).astype(np.float32)
     n = len(lens)
     S = (rng.standard_normal((n, H, 64, 64)) * 0.1).astype(np.float32)
+    if kind == "inf_s":
+        S[:, 1, 5, 9] = np.inf
     st = be.tensor(np.concatenate([[0], np.cumsum(lens)[:-1]]).astype(np.uint32), dtype=rsv.U32)
     ln = be.tensor(np.array(lens, np.uint32), dtype=rsv.U32)
     sl = be.tensor(np.arange(n, dtype=np.uint32)[::-1].copy(), dtype=rsv.U32)
@@ -483,9 +488,10 @@ def test_wkv7_seq_chunked_matches_token_by_token(be, kind, form, monkeypatch):
         out.append((be.get(yg, T * C), be.get(s2, S.size)))
     for (got, want), tol in zip(zip(out[1], out[0]), (2e-3, 1e-5)):
         fine = np.isfinite(want)
-        if kind in ("nan_k", "inf_v"):
+        if kind in ("nan_k", "inf_v", "inf_v_last", "inf_s"):
             assert not fine.all()
-        assert np.array_equal(fine, np.isfinite(got))
+        np.testing.assert_array_equal(got[~fine], want[~fine])  # the same infinities and NaNs
+        assert np.isfinite(got[fine]).all()
         assert rel_err(got[fine], want[fine]) < tol
 
 

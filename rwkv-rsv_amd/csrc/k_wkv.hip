@@ -1050,6 +1050,13 @@ __device__ __forceinline__ void lds_barrier() {
     __builtin_amdgcn_s_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
+// LDS passed from lane to lane of one wave: its LDS operations run in order, and
+// this keeps the compiler from reordering them (no instruction)
+__device__ __forceinline__ void lds_wave_order() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
+}
 
 // One lane's part of a chunk in flight: tokens 4(l/16) .. +3, columns 4(l%16) .. +3.
 struct WkvTok {
@@ -1143,6 +1150,7 @@ __device__ __forceinline__ int mm_prepare(WkvChunk &c, WkvTok &x, uint32_t nt, i
         *(f4_t *)&c.p[o2] = kk[i] * rs;
     }
     if (g == 0) *(f4_t *)&c.dec[4 * l16] = sg;
+    lds_wave_order();
     // A and Bm as four chains of 16 columns, added as a tree (they reach the state)
     f4_t gaq[4], gbq[4], gy = {0, 0, 0, 0}, gz = gy;
 #pragma unroll
@@ -1186,6 +1194,7 @@ __device__ __forceinline__ int mm_prepare(WkvChunk &c, WkvTok &x, uint32_t nt, i
         gy[e] = s16 <= t ? gy[e] : 0.0f;
         gz[e] = s16 <= t ? gz[e] : 0.0f;
     }
+    lds_wave_order();
     // P and G row by row (lane = column; G's 16 columns in every group), the
     // next row of A read ahead
     float gk[16], gg[16];
@@ -1218,7 +1227,7 @@ __device__ __forceinline__ int mm_prepare(WkvChunk &c, WkvTok &x, uint32_t nt, i
         for (int s4 = 0; s4 < (t + 4) / 4; s4++) at[s4] = an[s4];
         __builtin_amdgcn_sched_barrier(0);
     }
-    // (the reads of m are done: LDS operations of a wave are in order)
+    lds_wave_order();  // the reads of m go before the writes that replace it
 #pragma unroll
     for (int t = 0; t < 16; t++) c.p[mm_row(t) * kMmLd + lane] = gk[t];
     if (g == 0) {

@@ -687,10 +687,12 @@ __device__ __forceinline__ void block_sums(float (&v)[N], float (*red)[N]) {
 // are loaded at entry and their statistics taken together (two barriers a
 // block, where one pair of sums after another took four), so with R = 2 a row is
 // normalised once where its successor is in the block, and gamma, beta and the
-// mix coefficients are read once for both.  Rows of 2560 with one output: 4096
-// rows 30 -> 20 us (63 MB), 1500 12.8 -> 7.4, 700 6.5 -> 5.5; with six: 4096 43
-// -> 37 us (168 MB, 4.5 TB/s), 1500 19.6 -> 14.4, 700 10.5 -> 9.1.
-template <int R, int NT>
+// mix coefficients are read once for both.  EARLY loads the coefficients at entry
+// too: 48 more registers (112 : 60 with R = 1) for one latency less.
+// Against one pair of sums after another, rows of 2560: one output 4096 rows
+// 31 -> 19.5 us (63 MB), 1500 13.4 -> 7.7; six 4096 42 -> 34 us (168 MB, 4.9 TB/s),
+// 1500 19.8 -> 15.0, 256 5.9 -> 5.9.
+template <int R, int NT, bool EARLY>
 __global__ __launch_bounds__(NT) void k_seq_norm_mix(const float *__restrict__ x, const float *__restrict__ state,
                                                      const float *__restrict__ gamma, const float *__restrict__ beta,
                                                      Ptr6 coef, HOut6 out, int nout, const uint32_t *__restrict__ row_prev,
@@ -704,7 +706,7 @@ __global__ __launch_bounds__(NT) void k_seq_norm_mix(const float *__restrict__ x
     for (int i = 0; i < R; i++) p[i] = row_prev[min(t0 + i, T - 1)];
     // v[0]: the row before row t0 (raw x, or the slot's LN'd state row), v[1 + i]: row t0 + i
     const bool first_state = (p[0] & 0x80000000u) != 0;
-    float v[R + 1][kLnVec] = {}, gm[kLnVec] = {}, bt[kLnVec] = {};
+    float v[R + 1][kLnVec] = {}, gm[kLnVec] = {}, bt[kLnVec] = {}, cf[6][kLnVec];
     if (live) {
         if (!first_state) ld8(x + (size_t)p[0] * C + c0, v[0]);
         else if ((p[0] & 0x7FFFFFFFu) < slots) ld8(state + (size_t)(p[0] & 0x7FFFFFFFu) * C + c0, v[0]);
@@ -712,6 +714,9 @@ __global__ __launch_bounds__(NT) void k_seq_norm_mix(const float *__restrict__ x
         for (int i = 0; i < R; i++) ld8(x + (size_t)min(t0 + i, T - 1) * C + c0, v[1 + i]);
         ld8(gamma + c0, gm);
         ld8(beta + c0, bt);
+#pragma unroll
+        for (int j = 0; j < 6; j++)
+            if (EARLY && j < nout) ld8(coef.p[j] + c0, cf[j]);
     }
     float s[R + 1], q[R + 1];
 #pragma unroll
@@ -762,14 +767,13 @@ __global__ __launch_bounds__(NT) void k_seq_norm_mix(const float *__restrict__ x
 #pragma unroll
         for (int j = 0; j < 6; j++) {
             if (j >= nout) break;
-            float cf[kLnVec];
-            ld8(coef.p[j] + c0, cf);
+            if (!EARLY) ld8(coef.p[j] + c0, cf[j]);
             typedef _Float16 h8 __attribute__((ext_vector_type(8)));
             h8 o;
 #pragma unroll
             for (int e = 0; e < kLnVec; e++) {
                 const float a = v[1 + i][e], b = other ? alt[e] : v[i][e];
-                o[e] = (_Float16)(a + cf[e] * (b - a));
+                o[e] = (_Float16)(a + cf[j][e] * (b - a));
             }
             *(h8 *)(out.p[j] + (size_t)(t0 + i) * C + c0) = o;
         }
@@ -788,14 +792,24 @@ int launch_seq_norm_mix(rsv_ctx *ctx, const float *x, const float *state, const 
     HOut6 op{};
     for (int j = 0; j < nout; j++) { cp.p[j] = coef[j]; op.p[j] = out[j]; }
     const int nt = ln_threads(c), cus = ctx->sm_count > 0 ? ctx->sm_count : 256;
-#define SNM_LAUNCH(R, NT)                                                                                             \
-    hipLaunchKernelGGL((k_seq_norm_mix<R, NT>), dim3((t + (R) - 1) / (R)), dim3(nt), 0, ctx->stream, x, state, gamma, \
-                       beta, cp, op, nout, row_prev, t, c, slots, eps)
-    // two rows a block from four rows per CU on (1500 rows of 2560, one output,
-    // 8.9 us with one and 7.4 with two; 700 rows 5.5 and 5.7; four rows a block
-    // gained nothing at 4096 and lost below)
-    if (nt <= 512 && t >= 4 * cus) SNM_LAUNCH(2, 512);
-    else SNM_LAUNCH(1, 1024);
+#define SNM_LAUNCH(R, NT, EARLY)                                                                                      \
+    hipLaunchKernelGGL((k_seq_norm_mix<R, NT, EARLY>), dim3((t + (R) - 1) / (R)), dim3(nt), 0, ctx->stream, x, state, \
+                       gamma, beta, cp, op, nout, row_prev, t, c, slots, eps)
+    // Two rows a block once there are enough of them to keep the CUs busy: blocks
+    // of one or two waves from five rows per CU on (six outputs, one row a block :
+    // two, 1024 rows of 256 4.4 : 4.8 us, 1500 5.1 : 5.1, of 1024 8.2 : 7.8), larger
+    // ones from three and a half (1024 rows of 2048 10.9 : 9.8, 700 8.3 : 8.1).
+    // The coefficients of several outputs at entry where the launch is short or a
+    // block has one wave per SIMD at most (16 rows of 768, at use : at entry, 4.4 :
+    // 3.9 us, 1500 of 1024 8.7 : 7.8, 4096 of 2048 26.2 : 26.2); not for larger
+    // blocks with more rows than CUs, where the registers cost waves in flight (2560
+    // columns: 256 rows 6.2 : 5.9, 300 6.7 : 7.2, 1500 15.0 : 18.5, 4096 34 : 42).
+    const bool two = nt <= 512 && 2 * t >= (nt <= 128 ? 10 : 7) * cus;
+    const bool early = nout > 1 && (nt <= 256 || t <= (nt <= 512 ? cus : cus / 2));
+    if (early && two) SNM_LAUNCH(2, 256, true);  // (with more rows than CUs nt is at most 256)
+    else if (early) SNM_LAUNCH(1, 1024, true);
+    else if (two) SNM_LAUNCH(2, 512, false);
+    else SNM_LAUNCH(1, 1024, false);
 #undef SNM_LAUNCH
     RSV_HIP(hipGetLastError());
     return 0;

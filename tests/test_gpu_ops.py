@@ -365,10 +365,11 @@ def test_wkv7_seq_ragged_gate_matches_scan_times_gate(be, lens, scan_g, monkeypa
     assert rel_err(be.get(S2, S.size), be.get(S1, S.size)) < 1e-5
 
 
-@pytest.mark.parametrize("T,c,nout", [(1, 264, 1), (1023, 264, 6), (1024, 264, 1), (1027, 264, 6), (1030, 8192, 1)])
+@pytest.mark.parametrize("T,c,nout", [(1, 264, 1), (1023, 264, 6), (1024, 264, 1), (1027, 264, 6), (1030, 8192, 1), (255, 2568, 6), (897, 2568, 6),
+                                      (300, 4104, 2), (897, 2048, 6), (1281, 1024, 6), (1281, 264, 1)])
 def test_seq_norm_mix_rows(be, T, c, nout):
-    """rsv_seq_norm_mix below and from the row count where a block takes two
-    rows: an odd last row, segments that start on a block's first and second
+    """rsv_seq_norm_mix below and from the row counts where a block takes two
+    rows and where it reads the coefficients early or late: an odd last row, segments that start on a block's first and second
     row (from a state slot, one of them out of range: zeros), and a row whose
     predecessor is some other row.  fp16 outputs: 2^-11 relative, plus the LN's
     fp32 sums."""

@@ -665,10 +665,15 @@ __device__ __forceinline__ void gemmd_body(const GemmArgs &g, int m0, int n0, un
     // s + NS - 1: at steps 0 .. 3 of stage s (D = 1) or steps 2, 3 of it and
     // 0, 1 of stage s + 1 (D = 2; `late`).
     constexpr int NS = C::NS, D = C::D;
-#pragma unroll
-    for (int i = 0; i < NS - 1; i++) issue(i, i);
     static_assert((NS - 2) * NI < 63, "copies in flight fit the wait counter");
-    sk_wait_vm((NS - 2) * NI);
+    if (nst == 1) {  // k = 64: no copies of empty stages (4096 x 768 x 64 7.0 -> 6.6 us)
+        issue(0, 0);
+        sk_wait_vm(0);
+    } else {
+#pragma unroll
+        for (int i = 0; i < NS - 1; i++) issue(i, i);
+        sk_wait_vm((NS - 2) * NI);
+    }
     __builtin_amdgcn_s_barrier();
     u4 fa[4][MI], fb[4][NJ];
 #pragma unroll

@@ -499,8 +499,9 @@ int rsv_lane_record(rsv_ctx *ctx, int ev);
 int rsv_lane_wait(rsv_ctx *ctx, int lane, int ev);
 
 /* ---- raw access for harnesses: device pointer and stream of a tensor/ctx.
- * rsv_tensor_ptr waits for the context's stream (outside graph capture), so
- * that a new tensor's zero fill cannot land on what another stream writes. */
+ * The first rsv_tensor_ptr of a tensor (outside graph capture) waits for the
+ * stream that the tensor was created on, so that its zero fill cannot land on
+ * what another stream writes; later ones do not wait. */
 int rsv_tensor_ptr(rsv_ctx *ctx, uint32_t id, void **ptr);
 int rsv_stream(rsv_ctx *ctx, void **stream);
 

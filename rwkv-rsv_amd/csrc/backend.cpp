@@ -230,6 +230,7 @@ int rsv_tensor_create(rsv_ctx *ctx, uint64_t len, int dtype, uint32_t *id) {
     t.mem->ptr = t.ptr;
     t.mem->device = ctx->device;
     RSV_HIP(hipMemsetAsync(t.ptr, 0, (bytes + 63) & ~(size_t)63, ctx->stream));
+    t.fill = ctx->stream;
     t.live = true;
     if (!ctx->free_ids.empty()) {
         *id = ctx->free_ids.back();
@@ -283,9 +284,12 @@ int rsv_tensor_len(rsv_ctx *ctx, uint32_t id, uint64_t *len, int *dtype) {
 int rsv_tensor_ptr(rsv_ctx *ctx, uint32_t id, void **ptr) {
     Tensor *t = get_tensor(ctx, id);
     if (!t) return RSV_FAIL("tensor_ptr: unknown tensor id %u", id);
-    // a new tensor's zero fill is on the context's stream: done before another
-    // stream (the pointer's likely user) can write the tensor
-    if (!ctx->capturing && !ctx->prefill_capturing) RSV_HIP(hipStreamSynchronize(ctx->stream));
+    // a new tensor's zero fill is done before another stream (the pointer's likely
+    // user) can write the tensor: waited for once, on the lane it was issued on
+    if (t->fill && !ctx->capturing && !ctx->prefill_capturing) {
+        RSV_HIP(hipStreamSynchronize(t->fill));
+        t->fill = nullptr;
+    }
     *ptr = t->ptr;
     return 0;
 }
@@ -399,6 +403,7 @@ int rsv_import_tensors(rsv_ctx *ctx, rsv_ctx *src) {
     ctx->tensors.reserve(src->tensors.size());
     for (size_t i = 0; i < src->tensors.size(); i++) {
         Tensor t = src->tensors[i];
+        t.fill = nullptr;  // the source's matter: its streams may end before this context
         if (t.live) t.foreign = true;
         else {
             t = Tensor();

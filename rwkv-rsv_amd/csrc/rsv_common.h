@@ -43,6 +43,7 @@ struct Tensor {
     int dtype = RSV_F32;
     bool live = false;
     bool foreign = false;  // imported from another context (same id and memory as there)
+    hipStream_t fill = nullptr;  // the stream (lane) of the zero fill, until rsv_tensor_ptr has waited for it
     std::shared_ptr<DevMem> mem;
 };
 

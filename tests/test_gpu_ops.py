@@ -365,6 +365,41 @@ def test_wkv7_seq_ragged_gate_matches_scan_times_gate(be, lens, scan_g, monkeypa
     assert rel_err(be.get(S2, S.size), be.get(S1, S.size)) < 1e-5
 
 
+@pytest.mark.parametrize("created_on", [0, 1])
+def test_tensor_ptr_waits_for_the_zero_fill_only(be, created_on):
+    """The first pointer of a new tensor waits for its zero fill, on whichever
+    lane that was issued; further pointers do not wait for queued work."""
+    import torch
+    lib, m, n, k = _rsv().hip_lib(), 4096, 10240, 2560
+    a, w = be.tensor(n=m * k, dtype=_rsv().F16), be.tensor(n=n * k, dtype=_rsv().F16)
+    out = [be.tensor(n=m * n) for _ in range(2)]
+    ptr = ctypes.c_void_p()
+    be.call("rsv_tensor_ptr", a, ctypes.byref(ptr))
+    events = []
+    for lane in (0, 1):  # some 20 ms of work on either lane, so that nothing is done by itself
+        be.call("rsv_lane_select", lane)
+        be.call("rsv_stream", ctypes.byref(ptr))
+        stream = torch.cuda.ExternalStream(ptr.value)
+        be.call("rsv_gemm_ex", a, w, None, out[lane], m, n, k, 0, NONE, NONE, NONE)
+        torch.cuda.synchronize()
+        for _ in range(100):
+            be.call("rsv_gemm_ex", a, w, None, out[lane], m, n, k, 0, NONE, NONE, NONE)
+        events.append(torch.cuda.Event())
+        events[-1].record(stream)
+    be.call("rsv_tensor_ptr", a, ctypes.byref(ptr))
+    late = [e.query() for e in events]
+    new = ctypes.c_uint32()
+    be.call("rsv_lane_select", created_on)
+    be.call("rsv_tensor_create", 1 << 20, _rsv().F32, ctypes.byref(new))
+    be.call("rsv_lane_select", 1 - created_on)
+    be.call("rsv_tensor_ptr", new, ctypes.byref(ptr))
+    done = events[created_on].query()
+    be.call("rsv_lane_select", 0)
+    torch.cuda.synchronize()
+    lib.rsv_tensor_free(be.ctx, new)
+    assert late[1] is False and done
+
+
 @pytest.mark.parametrize("T,c,nout", [(1, 264, 1), (1023, 264, 6), (1024, 264, 1), (1027, 264, 6), (1030, 8192, 1), (255, 2568, 6), (897, 2568, 6),
                                       (300, 4104, 2), (897, 2048, 6), (1281, 1024, 6), (1281, 264, 1)])
 def test_seq_norm_mix_rows(be, T, c, nout):

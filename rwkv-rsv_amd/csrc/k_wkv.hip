@@ -832,8 +832,8 @@ int launch_wkv7_seq_ragged(rsv_ctx *ctx, float *s, const float *r, const float *
 
 // ------------------------------------- ragged prefill scan, gated fp16 out
 // The scan of rsv_wkv7_seq_ragged_gate, leaving the att.output operand
-// yg = (GroupNorm(y) + bonus*v) * g in fp16: a scan (k_wkv7_seq_mm 16 tokens at
-// a time, k_wkv7_seq_cols token by token for short segments) writes the raw
+// yg = (GroupNorm(y) + bonus*v) * g in fp16: a scan (k_wkv7_seq_mm 16 tokens at a
+// time, k_wkv7_seq_cols and _rows token by token for short segments) writes the raw
 // y = S r and the head's bonus sum per token, then k_gn_gate_f16 applies
 // GroupNorm + bonus*v and the gate.
 //
@@ -954,6 +954,160 @@ __global__ __launch_bounds__(512) void k_wkv7_seq_cols(
         ((float4 *)Sr)[m] = make_float4(s[4 * m], s[4 * m + 1], s[4 * m + 2], s[4 * m + 3]);
 }
 
+// Token by token with RPL state rows per group of four lanes, 64 / RPL groups per
+// (head, segment): fewer LDS reads of the head's vectors per state row than the
+// form above and fewer waves per block, at a longer chain per token.  For launches
+// of many short segments whose inputs are past the cache (see the launcher); the
+// first nlong segments of at least long_len tokens are left to k_wkv7_seq_mm.  The
+// reductions over the head are formed four tokens per wave.
+template <int RPL>
+__global__ __launch_bounds__(256 / RPL) void k_wkv7_seq_rows(
+    float *__restrict__ S, const float *__restrict__ r, const float *__restrict__ w, const float *__restrict__ k,
+    const float *__restrict__ v, const float *__restrict__ a, const float *__restrict__ kkc,
+    const float *__restrict__ ka, const float *__restrict__ rk, float *__restrict__ y_out,
+    float *__restrict__ bonus_out, const uint32_t *__restrict__ seg_start, const uint32_t *__restrict__ seg_len,
+    const uint32_t *__restrict__ seg_slot, int H, float eps, uint64_t rows, uint64_t slots, uint32_t long_len,
+    uint32_t nlong) {
+    constexpr int NW = 4 / RPL;   // waves per (head, segment)
+    constexpr int kRB = 4 * NW;   // tokens per batch: four per wave in the batch phase
+    // per batch: [token][k^ | -k^ a | w | k_mod | r | v] x 64 columns, two batches alternating
+    __shared__ __attribute__((aligned(16))) float hb[2][kRB][6 * 64];
+    // the batch's outputs (y per token and row, the bonus sum per token) are
+    // staged in LDS and stored once the batch is done: a global store per
+    // token would hold its data register until the write completes
+    __shared__ __attribute__((aligned(16))) float yl[2][kRB][64];
+    __shared__ float bl[2][kRB];
+    const int h = blockIdx.x, gi = blockIdx.y, tid = threadIdx.x;
+    const int wave = tid >> 6, lane = tid & 63, q = lane & 3;
+    const int row0 = 16 * RPL * wave + RPL * (lane >> 2);  // this lane's rows row0 .. row0 + RPL - 1
+    const size_t C = (size_t)H * 64;
+    const uint32_t t0 = seg_start[gi], len = seg_len[gi], slot = seg_slot[gi];
+    if (slot >= slots || (uint64_t)t0 + len > rows) return;  // uniform per block
+    if (len >= long_len) {  // taken by k_wkv7_seq_mm, if it is among the first nlong of them
+        uint32_t before = 0;
+        for (int b = 0; b < gi; b += 64) before += (uint32_t)__popcll(__ballot(b + lane < gi && seg_len[min(b + lane, gi)] >= long_len));
+        if (before < nlong) return;
+    }
+    float4 *Sb = (float4 *)(S + ((size_t)slot * H + h) * 4096);
+    float s[RPL][16];
+#pragma unroll
+    for (int i = 0; i < RPL; i++)
+#pragma unroll
+        for (int m = 0; m < 4; m++) {
+            const float4 x = Sb[(row0 + i) * 16 + 4 * q + m];
+            s[i][4 * m] = x.x; s[i][4 * m + 1] = x.y; s[i][4 * m + 2] = x.z; s[i][4 * m + 3] = x.w;
+        }
+    // column role (batch phase): lane j forms column j's vectors of tokens
+    // 4*wave .. 4*wave+3 of a batch; every reduction over the head happens
+    // here, for four tokens at once, off the scan's dependent chain
+    const int j = lane;
+    const float kkc_j = kkc[h * 64 + j], ka_j = ka[h * 64 + j], rk_j = rk[h * 64 + j];
+    float pk[4], pa[4], pw[4], pr[4], pv[4];
+    auto load_batch = [&](uint32_t tb) {
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const uint32_t t = tb + 4 * wave + i;
+            const size_t vo = (size_t)(t0 + (t < len ? t : 0)) * C + (size_t)h * 64 + j;
+            pk[i] = k[vo]; pa[i] = a[vo]; pw[i] = w[vo]; pr[i] = r[vo]; pv[i] = v[vo];
+        }
+    };
+    auto form_batch = [&](int buf, uint32_t tb) {
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const uint32_t t = tb + 4 * wave + i;
+            if (t >= len) break;  // uniform per wave
+            const float kc = pk[i], ac = pa[i], rc = pr[i];
+            const float kk = kc * kkc_j;
+            float nrm = sqrtf(wave_sum(kk * kk));
+            nrm = nrm < eps ? eps : nrm;
+            const float kh = kk * (1.0f / nrm);
+            const float kmod = kc + ka_j * (kc * ac - kc);
+            const float bonus = wave_sum(rc * kmod * rk_j);
+            float *hv = hb[buf][4 * wave + i];
+            hv[j] = kh; hv[64 + j] = kh * (-ac); hv[128 + j] = pw[i]; hv[192 + j] = kmod; hv[256 + j] = rc; hv[320 + j] = pv[i];
+            if (j == 0) bl[buf][4 * wave + i] = bonus;
+        }
+    };
+    auto flush = [&](int buf, uint32_t tb) {
+        // kRB tokens x 64 rows = one float4 per thread (non-temporal: acknowledged sooner)
+        typedef float f4v __attribute__((ext_vector_type(4)));
+        const uint32_t u = tid >> 4, c4 = 4 * (tid & 15);
+        if (tb + u < len) {
+            const float4 yv = *(const float4 *)&yl[buf][u][c4];
+            __builtin_nontemporal_store((f4v){yv.x, yv.y, yv.z, yv.w}, (f4v *)(y_out + (size_t)(t0 + tb + u) * C + (size_t)h * 64 + c4));
+        }
+        if (tid < kRB && tb + tid < len) __builtin_nontemporal_store(bl[buf][tid], bonus_out + (size_t)(t0 + tb + tid) * H + h);
+    };
+    if (len > 0) {
+        load_batch(0);
+        form_batch(0, 0);
+    }
+    for (uint32_t tb = 0; tb < len; tb += kRB) {
+        const int buf = (tb / kRB) & 1;
+        // the batch's vectors are in LDS (lgkmcnt(0), then the barrier); the
+        // other buffer is free
+        __builtin_amdgcn_s_waitcnt(0xC07F);
+        __builtin_amdgcn_s_barrier();
+        if (tb > 0) flush(buf ^ 1, tb - kRB);  // the previous batch's outputs
+        const bool more = tb + kRB < len;
+        if (more) load_batch(tb + kRB);  // in flight during the scan below
+        const uint32_t nt = len - tb < (uint32_t)kRB ? len - tb : (uint32_t)kRB;
+        for (uint32_t u = 0; u < nt; u++) {
+            const float *hv = hb[buf][u];
+            float kv[16], bv[16], wv[16], mv[16], rv[16], vc[RPL];
+#pragma unroll
+            for (int m = 0; m < 4; m++) {
+                const float4 a0 = *(const float4 *)(hv + 16 * q + 4 * m), a1 = *(const float4 *)(hv + 64 + 16 * q + 4 * m),
+                             a2 = *(const float4 *)(hv + 128 + 16 * q + 4 * m), a3 = *(const float4 *)(hv + 192 + 16 * q + 4 * m),
+                             a4 = *(const float4 *)(hv + 256 + 16 * q + 4 * m);
+                kv[4 * m] = a0.x; kv[4 * m + 1] = a0.y; kv[4 * m + 2] = a0.z; kv[4 * m + 3] = a0.w;
+                bv[4 * m] = a1.x; bv[4 * m + 1] = a1.y; bv[4 * m + 2] = a1.z; bv[4 * m + 3] = a1.w;
+                wv[4 * m] = a2.x; wv[4 * m + 1] = a2.y; wv[4 * m + 2] = a2.z; wv[4 * m + 3] = a2.w;
+                mv[4 * m] = a3.x; mv[4 * m + 1] = a3.y; mv[4 * m + 2] = a3.z; mv[4 * m + 3] = a3.w;
+                rv[4 * m] = a4.x; rv[4 * m + 1] = a4.y; rv[4 * m + 2] = a4.z; rv[4 * m + 3] = a4.w;
+            }
+#pragma unroll
+            for (int i = 0; i < RPL; i++) vc[i] = hv[320 + row0 + i];
+            float sa[RPL], y[RPL];
+#pragma unroll
+            for (int i = 0; i < RPL; i++) {
+                sa[i] = 0.f;
+#pragma unroll
+                for (int e = 0; e < 16; e++) sa[i] = fmaf(s[i][e], kv[e], sa[i]);
+            }
+#pragma unroll
+            for (int i = 0; i < RPL; i++) sa[i] = quad_sum(sa[i]);
+#pragma unroll
+            for (int i = 0; i < RPL; i++) {
+                y[i] = 0.f;
+#pragma unroll
+                for (int e = 0; e < 16; e++) {
+                    const float ns = s[i][e] * wv[e] + sa[i] * bv[e] + vc[i] * mv[e];
+                    s[i][e] = ns;
+                    y[i] = fmaf(ns, rv[e], y[i]);
+                }
+            }
+#pragma unroll
+            for (int i = 0; i < RPL; i++) y[i] = quad_sum(y[i]);
+            if (q == 0)
+#pragma unroll
+                for (int i = 0; i < RPL; i++) yl[buf][u][row0 + i] = y[i];
+        }
+        if (more) form_batch(buf ^ 1, tb + kRB);
+    }
+    if (len > 0) {
+        __builtin_amdgcn_s_waitcnt(0xC07F);
+        __builtin_amdgcn_s_barrier();
+        const uint32_t last = (len - 1) / kRB * kRB;
+        flush((last / kRB) & 1, last);
+    }
+#pragma unroll
+    for (int i = 0; i < RPL; i++)
+#pragma unroll
+        for (int m = 0; m < 4; m++)
+            Sb[(row0 + i) * 16 + 4 * q + m] = make_float4(s[i][4 * m], s[i][4 * m + 1], s[i][4 * m + 2], s[i][4 * m + 3]);
+}
+
 // ------------------------------- chunked scan on matrix cores (fp32 MFMA)
 // The same recurrence, 16 tokens at a time.  With sigma_t the product of the
 // decays of the tokens after t in the chunk (per column; sigma_15 = 1),
@@ -975,8 +1129,7 @@ __global__ __launch_bounds__(512) void k_wkv7_seq_cols(
 // decays fp64); the state's error against 64 bits is below that of the
 // token-by-token scan: decays drawn per token 6.8e-8 : 7.2e-8 at every shape from
 // 1 x 40 to 24 segments of 4096.  Two things keep it there, sigma from 64 bits and
-// the order of the state's sums; with neither it was 8.1e-8 to 8.9e-8 (and 2 % of
-// the scan's time faster: 5 x 512 at 40 heads 99 -> 101 us).
+// the order of the state's sums; with neither it was 8.1e-8 to 8.9e-8.
 //   - S is held transposed in the MFMA accumulator layout: lane l, register
 //     (q, e) is S[row = l%16][column = 16q + 4(l/16) + e].  As the B operand of
 //     k-step (q, e) it is used in place: the four k of a step may be any four
@@ -1385,6 +1538,29 @@ __device__ __forceinline__ bool mm_wild(const f4_t (&s)[4]) {
     return __ballot(!fine) != 0;
 }
 
+// The n-th segment of at least min_len tokens, or -1 (per wave).
+__device__ __forceinline__ int nth_long(const uint32_t *__restrict__ seg_len, int nseg, uint32_t min_len, uint32_t n, int lane) {
+    for (int b = 0; b < nseg; b += 256) {
+        uint64_t m[4];
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const int j = b + 64 * i + lane;
+            const uint32_t len = seg_len[min(j, nseg - 1)];
+            m[i] = __ballot(j < nseg && len >= min_len);
+        }
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const uint32_t k = (uint32_t)__popcll(m[i]);
+            if (n < k) {
+                for (; n > 0; n--) m[i] &= m[i] - 1;
+                return b + 64 * i + __ffsll((unsigned long long)m[i]) - 1;
+            }
+            n -= k;
+        }
+    }
+    return -1;
+}
+
 // One block per (head, segment, 4/NC-th of its rows): waves NC.. prepare the
 // next NP chunks, one each, into one set while waves 0..NC-1 pass the state's
 // rows, 16 each, through the NP chunks of the other.
@@ -1400,12 +1576,16 @@ __global__ __launch_bounds__(512, 2) void k_wkv7_seq_mm(
     const float *__restrict__ v, const float *__restrict__ a, const float *__restrict__ kkc,
     const float *__restrict__ ka, const float *__restrict__ rk, float *__restrict__ y_out,
     float *__restrict__ bonus_out, const uint32_t *__restrict__ seg_start, const uint32_t *__restrict__ seg_len,
-    const uint32_t *__restrict__ seg_slot, int H, float eps, uint64_t rows, uint64_t slots) {
+    const uint32_t *__restrict__ seg_slot, int H, float eps, uint64_t rows, uint64_t slots,
+    int nseg, uint32_t min_len) {
     __shared__ __attribute__((aligned(16))) WkvChunk chunk[2][NP];
     constexpr uint32_t kSup = 16 * NP;  // tokens of a superstep
-    const int h = blockIdx.x, gi = blockIdx.y, tid = threadIdx.x;
+    const int h = blockIdx.x, tid = threadIdx.x;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, l16 = lane & 15, g = lane >> 4;
     const size_t C = (size_t)H * 64;
+    // with min_len, the blockIdx.y-th of the segments that long
+    const int gi = min_len ? nth_long(seg_len, nseg, min_len, blockIdx.y, lane) : (int)blockIdx.y;
+    if (gi < 0) return;  // uniform per block
     const uint32_t t0 = seg_start[gi], len = seg_len[gi], slot = seg_slot[gi];
     if (slot >= slots || (uint64_t)t0 + len > rows || len == 0) return;  // uniform per block
     const uint32_t nsup = (len + kSup - 1) / kSup;
@@ -1531,28 +1711,51 @@ int launch_wkv7_seq_ragged_gate(rsv_ctx *ctx, float *s, const float *r, const fl
     if (n != 64) return RSV_FAIL("wkv7_seq: head_size must be 64 (got %d)", n);
     if (nseg <= 0 || rows == 0) return 0;
     {
-#define WKV_MM_LAUNCH(NC, NP)                                                                                         \
-    hipLaunchKernelGGL((k_wkv7_seq_mm<NC, NP>), dim3(h, nseg, 4 / (NC)), dim3(64 * ((NC) + (NP))), 0, ctx->stream, s, r, \
-                       w, k, v, a, kk, ka, rk, y_work, bonus_work, seg_start, seg_len, seg_slot, h, 1e-12f, rows, slots)
-        // The chunked scan from 24 tokens a segment on (the mean: the lengths are
-        // on the device), from 48 where the blocks take more than two rounds over
-        // the CUs (one block per CU; k_wkv7_seq_cols packs several).  40 heads,
-        // scan and GroupNorm pass, us against the token-by-token form taken for
-        // the shape before: 1 x 700 tokens 96 : 219, 8 x 512 191 : 448, 24
-        // segments of 4096 178 : 287, 64 of 4096 206 : 236, 32 x 512 600 : 837.
-        // Near the line, against k_wkv7_seq_cols: 1 x 40 16 : 19, 10 x 32 28 : 33,
-        // 5 x 20 16 : 16, 10 x 16 25 : 21; 24 x 43 63 : 60, 64 x 32 133 : 115.
-        // A quarter of a head's rows per block while every block still has a CU:
-        // 1 x 700 96 against 109.  RSV_SCAN_G selects a form: 4 and 1 heads per
-        // whole or quarter block, anything else token by token.
+#define WKV_MM_LAUNCH(NC, NP, Y, MIN)                                                                                 \
+    hipLaunchKernelGGL((k_wkv7_seq_mm<NC, NP>), dim3(h, Y, 4 / (NC)), dim3(64 * ((NC) + (NP))), 0, ctx->stream, s, r, w, \
+                       k, v, a, kk, ka, rk, y_work, bonus_work, seg_start, seg_len, seg_slot, h, 1e-12f, rows, slots,  \
+                       nseg, MIN)
+#define WKV_ROWS_LAUNCH(R)                                                                                            \
+    hipLaunchKernelGGL(k_wkv7_seq_rows<R>, dim3(h, nseg), dim3(256 / (R)), 0, ctx->stream, s, r, w, k, v, a, kk, ka, rk, \
+                       y_work, bonus_work, seg_start, seg_len, seg_slot, h, 1e-12f, rows, slots, kLong, (uint32_t)most)
+        // All by the mean length (the lengths are on the device); us at 40 heads,
+        // scan and GroupNorm pass.
+        // The chunked scan from 24 tokens a segment on, from 64 where the blocks take
+        // more than two rounds over the CUs (one block per CU; k_wkv7_seq_cols packs
+        // several).  Against the token-by-token forms taken before it: 1 x 700 tokens 90
+        // : 219, 8 x 512 187 : 452, 24 x 128 119 : 161, 32 x 512 559 : 740.  Near the
+        // line, against k_wkv7_seq_cols: 1 x 40 16 : 21, 8 x 32 26 : 26, 5 x 20 15 : 14;
+        // 20 x 48 61 : 58, 64 x 48 151 : 133, 20 x 64 72 : 73, 32 x 64 94 : 92.
+        // A quarter of a head's rows per block while every block still has a CU: 1 x
+        // 512 71 against 83.
+        // Many short segments whose inputs are past the 256 MB cache are faster in
+        // k_wkv7_seq_rows (5 and 8 blocks a CU against 3), against k_wkv7_seq_cols 128 x
+        // 32 180 : 193, 256 x 16 205 : 210, 384 x 32 511 : 581; four rows per group past
+        // 500 MB (64 heads, 256 x 48, two : four 767 : 742).  Its longer chain per token
+        // is kept from long segments: those of kLong tokens on go to a chunked launch of
+        // their own (100 x 20 + 1 x 2000 399, in one form 741 to 1330; with no such
+        // segment it costs about 2 % of the whole).
+        // RSV_SCAN_G selects a form: 4 and 1 chunked with a head and a quarter of one
+        // per block, -2 and -4 k_wkv7_seq_rows, anything else k_wkv7_seq_cols.
+        constexpr uint32_t kLong = 256;
         const int blocks = h * nseg, cus = ctx->sm_count > 0 ? ctx->sm_count : 256;
+        const uint64_t bytes = rows * (uint64_t)h * (64 * 6 * 4), n = (uint64_t)nseg;
+        const bool past_cache = bytes >= 224u * 1000 * 1000 && blocks >= 12 * cus && rows >= 10 * n && rows < 96 * n;
         const char *e = getenv("RSV_SCAN_G");
-        const int gsel = e ? atoi(e) : rows < (blocks <= 2 * cus ? 24u : 48u) * (uint64_t)nseg ? 0 : blocks * 4 <= cus ? 1 : 4;
-        if (gsel == 4) WKV_MM_LAUNCH(4, 4);
-        else if (gsel == 1) WKV_MM_LAUNCH(1, 3);
-        else
+        const int gsel = e ? atoi(e)
+                           : past_cache ? (bytes >= 500u * 1000 * 1000 && blocks >= 16 * cus ? -4 : -2)
+                                        : rows < (blocks <= 2 * cus ? 24u : 64u) * n ? 0 : blocks * 4 <= cus ? 1 : 4;
+        if (gsel == 4) WKV_MM_LAUNCH(4, 4, nseg, 0u);
+        else if (gsel == 1) WKV_MM_LAUNCH(1, 3, nseg, 0u);
+        else if (gsel == -2 || gsel == -4) {
+            const int most = (int)std::min<uint64_t>(n, rows / kLong);
+            if (most > 0) WKV_MM_LAUNCH(4, 4, most, kLong);
+            if (gsel == -2) WKV_ROWS_LAUNCH(2);
+            else WKV_ROWS_LAUNCH(4);
+        } else
             hipLaunchKernelGGL(k_wkv7_seq_cols, dim3(h, nseg), dim3(512), 0, ctx->stream, s, r, w, k, v, a, kk, ka, rk, y_work,
                                bonus_work, seg_start, seg_len, seg_slot, h, 1e-12f, rows, slots);
+#undef WKV_ROWS_LAUNCH
 #undef WKV_MM_LAUNCH
         const uint64_t units = rows * (uint64_t)h;
         hipLaunchKernelGGL(k_gn_gate_f16, dim3((unsigned)((units + 15) / 16)), dim3(256), 0, ctx->stream, y_work,

@@ -328,15 +328,16 @@ def test_wkv7_seq_ragged_matches_decode_loop(be):
         pos += lens[g]
 
 
-@pytest.mark.parametrize("scan_g", ["", "16", "8", "0", "-4"])
-@pytest.mark.parametrize("lens", [[300, 212], [8] * 48 + [40], [512]])
+@pytest.mark.parametrize("scan_g", ["", "4", "1", "0", "-2", "-4"])
+@pytest.mark.parametrize("lens", [[300, 212], [8] * 48 + [40], [512], [1, 256, 20, 255, 64]])
 def test_wkv7_seq_ragged_gate_matches_scan_times_gate(be, lens, scan_g, monkeypatch):
-    """rsv_wkv7_seq_ragged_gate leaves (GroupNorm(y) + bonus*v) * g in fp16:
-    with few segments it runs the four-lanes-per-row scan and a separate
-    GroupNorm pass, with many the one-wave scan; both against
-    rsv_wkv7_seq_ragged's yn times g (and its state) to rounding.  scan_g
-    forces the scan form (16 or 8 lanes per state row, 0 the two-rows-per-
-    group form, -4 four rows per group; empty: chosen by the block count)."""
+    """rsv_wkv7_seq_ragged_gate leaves (GroupNorm(y) + bonus*v) * g in fp16, by
+    one of several scans and a separate GroupNorm pass; against the one-wave
+    scan of rsv_wkv7_seq_ragged (its yn times g, and its state) to rounding.
+    scan_g forces the form: 4 and 1 chunked with a whole head and a quarter of
+    one per block, 0 token by token with eight lanes per row, -2 and -4 with two
+    and four rows per group of lanes (segments of 256 tokens on chunked); empty:
+    chosen by the sizes."""
     rsv = _rsv()
     if scan_g:
         monkeypatch.setenv("RSV_SCAN_G", scan_g)
@@ -363,6 +364,36 @@ def test_wkv7_seq_ragged_gate_matches_scan_times_gate(be, lens, scan_g, monkeypa
     got = be.get(yg, T * C)
     assert rel_err(got, want) < 2e-3
     assert rel_err(be.get(S2, S.size), be.get(S1, S.size)) < 1e-5
+
+
+@pytest.mark.parametrize("form,H,lens,starts", [
+    ("-2", 2, [2] * 270 + [256, 300] + [3] * 27 + [257], None),  # long ones past the first 256 segments
+    ("-4", 2, [256] * 3 + [1] * 70 + [255, 700], None),
+    ("-2", 3, [300] * 3, [0] * 3),  # the same rows for three slots: more long segments than rows / 256
+    ("", 40, [300] + [7, 60, 33, 48] * 22 + [1, 120], None),  # chosen by the sizes: past the cache, many segments
+])
+def test_wkv7_seq_rows_and_long_segments(be, form, H, lens, starts, monkeypatch):
+    """k_wkv7_seq_rows beside the chunked launch that takes its long segments:
+    every segment once, whatever its index, against the form with eight lanes
+    per row (other sums' order: some hundred roundings of 2^-24)."""
+    rsv = _rsv()
+    C, n = H * 64, len(lens)
+    starts = np.concatenate([[0], np.cumsum(lens)[:-1]]) if starts is None else starts
+    T = int(max(s + m for s, m in zip(starts, lens)))
+    r, v, k, w, a, _, kk, ka, rk, gam, bet = _wkv_inputs(np.random.default_rng(n), T, H)
+    S = np.tile((np.random.default_rng(1).standard_normal((1, H, 64, 64)) * 0.1).astype(np.float32), (n, 1, 1, 1))
+    st, ln, sl = (be.tensor(np.asarray(z, np.uint32), dtype=rsv.U32) for z in (starts, lens, range(n)))
+    common = [be.tensor(z) for z in (r, w, k, v, a, kk, ka, rk, gam, bet)]
+    gt, yw, bw, yg = be.tensor(a), be.tensor(n=T * C), be.tensor(n=T * H), be.tensor(n=T * C, dtype=rsv.F16)
+    out = []
+    for which in ("0", form):
+        monkeypatch.setenv("RSV_SCAN_G", which) if which else monkeypatch.delenv("RSV_SCAN_G")
+        s2 = be.tensor(S)
+        be.call("rsv_wkv7_seq_ragged_gate", s2, *common, gt, yw, bw, yg, st, ln, sl, n, T, H, 64, 64e-5)
+        out.append((be.get(yg, T * C), be.get(s2, S.size)))
+        be.call("rsv_tensor_free", s2)
+    assert rel_err(out[1][0], out[0][0]) < 2e-3
+    assert rel_err(out[1][1], out[0][1]) < 1e-5
 
 
 @pytest.mark.parametrize("created_on", [0, 1])

@@ -468,12 +468,14 @@ def test_seq_norm_mix_rows(be, T, c, nout):
 
 
 @pytest.mark.parametrize("form", ["4", "1"])
-@pytest.mark.parametrize("decays", ["token", "channel"])
+@pytest.mark.parametrize("decays", ["token", "channel", "steep"])
 def test_wkv7_seq_chunked_state_error_against_64_bits(be, decays, form, monkeypatch):
     """The chunked scan may not lose precision: its state is no further from
     64 bits (2-norm) than the token-by-token form's, with decays drawn
-    for each token, where the last few tokens' roundings count, and decays of the
-    channel, where those of hundreds of tokens add up."""
+    for each token, where the last few tokens' roundings count, decays of the
+    channel, where those of hundreds of tokens add up; and within one rounding
+    with decays of 2^-32 a chunk, near the largest that the chunked form takes
+    (a model's are at most 2^-14)."""
     rsv = _rsv()
     H, lens = 4, [40, 200, 460]
     C, T, n = H * 64, sum(lens), len(lens)
@@ -481,6 +483,8 @@ def test_wkv7_seq_chunked_state_error_against_64_bits(be, decays, form, monkeypa
     r, v, k, _, a, _, kk, ka, rk, gam, bet = _wkv_inputs(rng, T, H)
     x = rng.standard_normal((T, C)) * 2 - 1.5 if decays == "token" else rng.standard_normal(C) * 2 - 1.5 + rng.standard_normal((T, C)) * 0.5
     w = np.exp(-0.6065 / (1 + np.exp(-x))).astype(np.float32)
+    if decays == "steep":
+        w = (0.25 + 0.14 * (rng.random((T, C)) - 0.5)).astype(np.float32)
     S = (rng.standard_normal((n, H, 64, 64)) * 0.1).astype(np.float32)
     starts = np.concatenate([[0], np.cumsum(lens)[:-1]])
     k64, v64, w64, a64 = (z.astype(np.float64).reshape(T, H, 64) for z in (k, v, w, a))
@@ -501,16 +505,19 @@ def test_wkv7_seq_chunked_state_error_against_64_bits(be, decays, form, monkeypa
         yg = be.tensor(n=T * C, dtype=rsv.F16)
         be.call("rsv_wkv7_seq_ragged_gate", s2, *common, gt, yw, bw, yg, st, ln, sl, n, T, H, 64, 64e-5)
         err.append(np.linalg.norm(be.get(s2, S.size) - want.reshape(-1)) / np.linalg.norm(want))
-    assert err[1] <= err[0], err
+    # steep: only the last tokens count, and each form's error is about the one
+    # rounding that the stored state cannot do without, at most half of 2^-23
+    assert err[1] <= (2.0 ** -24 if decays == "steep" else err[0]), err
 
 
 @pytest.mark.parametrize("form", ["4", "1"])
-@pytest.mark.parametrize("kind", ["model", "strong", "big", "over", "nan_k", "inf_v", "inf_v_last", "inf_s"])
+@pytest.mark.parametrize("kind", ["model", "strong", "big", "over", "nan_k", "inf_v", "inf_v_last", "inf_s", "steep", "past"])
 def test_wkv7_seq_chunked_matches_token_by_token(be, kind, form, monkeypatch):
     """The chunked scan (whole heads and quarters per block) against the
     token-by-token form, at segment lengths around its chunks of 16 and its
     supersteps of 48 and 64 tokens: decays of the model, decays down to 0 and
-    keys of 1e13 (both leave its range and are stepped token by token), finite
+    keys of 1e13 (both leave its range and are stepped token by token), decays
+    near the guard of 2^-40 a chunk, within it and past it, finite
     keys whose sum of squares overflows (k^ = 0, no NaN), and inputs or a state
     that are not finite, which must reach the same tokens and rows and leave the
     same infinities and NaNs.
@@ -526,6 +533,10 @@ def test_wkv7_seq_chunked_matches_token_by_token(be, kind, form, monkeypatch):
     if kind == "strong":
         w = rng.random((T, C)).astype(np.float32) ** 4
         w[rng.random((T, C)) < 0.02] = 0.0
+    elif kind == "steep":  # 2^-32 a chunk of 16 tokens on average, the steepest of a head's columns about 2^-37
+        w = (0.25 + 0.14 * (rng.random((T, C)) - 0.5)).astype(np.float32)
+    elif kind == "past":  # 2^-43
+        w = (0.155 + 0.02 * (rng.random((T, C)) - 0.5)).astype(np.float32)
     elif kind == "big":
         k, rk = k * np.float32(1e13), rk * 0  # (no bonus: it would leave fp16's range)
     elif kind == "over":
@@ -568,8 +579,8 @@ def test_wkv7_seq_config2_t512(be, nseg):
     through rsv_wkv7_seq_ragged, segments written to permuted state slots;
     three segments checked token by token against the oracle step (y every
     token, the final state), and the gated fp16 form of the prefill
-    (rsv_wkv7_seq_ragged_gate, the four-lanes-per-row scan at this segment
-    count) against yn * g and the same states."""
+    (rsv_wkv7_seq_ragged_gate, the chunked scan at this segment length)
+    against yn * g and the same states."""
     rsv = _rsv()
     H, L = 40, 512
     C, T = H * 64, nseg * 512
@@ -1064,11 +1075,11 @@ def test_gemm_prefill_shapes(be, m, n, k):
 @pytest.mark.parametrize("m,n,k", [(4096, 2560, 2560), (2048, 2560, 2560), (1024, 2560, 2560), (3000, 640, 10240),
                                    (1030, 384, 640)])
 def test_gemm_dma_tiles_equal_int8_loader(be, m, n, k):
-    """The fp16-weight prefill GEMM (operand tiles copied to LDS by DMA, one
-    of three tile shapes picked by the grid size: these shapes take each of
-    them, with partial tiles) on the fp16 copy of an int8 matrix gives the
-    int8 loader's results bit for bit (the same MFMA chain per element), and
-    both match float64 with the loader's fp16 rounding of the weights."""
+    """The fp16-weight prefill GEMM (operand tiles copied to LDS by DMA, the
+    tile picked by the grid size: here 256x160, 256x128, 128x128 and 64x64, with
+    partial tiles) on the fp16 copy of an int8 matrix gives the int8 loader's
+    results bit for bit (the same MFMA chain per element), and both match
+    float64 with the loader's fp16 rounding of the weights."""
     rsv = _rsv()
     rng = np.random.default_rng(m + 3 * n + k)
     A = rng.standard_normal((m, k)).astype(np.float16)
@@ -1091,7 +1102,8 @@ def test_gemm_dma_tiles_equal_int8_loader(be, m, n, k):
 @pytest.mark.parametrize("m,n", [(1, 64), (63, 100), (65, 2562), (129, 5120), (191, 10240), (517, 2560), (1000, 2560)])
 def test_gemm_dma_tiles_agree_bit_for_bit(be, m, n, k):
     """Few rows take the 64x64 and 64x128 tiles (then 128x128), many rows the
-    large ones: row r of an m-row product equals row r of the same product
+    large ones (with n up to 100 both are 64x64: see the test against the other
+    forms below): row r of an m-row product equals row r of the same product
     over a chip-filling batch, bit for bit (one MFMA chain per element), for
     every fill of the stage buffers (k / 64 from 1 up), n without the 16-byte
     epilogue included; and float64 within the fp32 accumulation bound."""
@@ -1111,6 +1123,33 @@ def test_gemm_dma_tiles_agree_bit_for_bit(be, m, n, k):
     A64, W64 = A[:m].astype(np.float64), W.astype(np.float64)
     bound = k * 2.0 ** -24 * (np.abs(A64) @ np.abs(W64).T)  # k additions of one rounding each
     assert np.all(np.abs(got - A64 @ W64.T) <= bound)
+
+
+@pytest.mark.parametrize("k", [64, 128, 192, 640])
+@pytest.mark.parametrize("m,ns", [
+    # one product: 64x64 tiles, 64x128, 128x128, 256x128, 256x160
+    (63, [64]), (64, [100]), (65, [2562]), (191, [10242]), (999, [2562]), (517, [10242]), (2050, [2562]), (2049, [7682]),
+    # lists: 64x64, 64x128, 128x128, 256x128, 256x160
+    (65, [2560, 2562, 96]), (301, [2560, 2562, 96]), (517, [2560, 2562, 96]), (1000, [2560, 2562, 96]), (3100, [2560, 2562, 96])])
+def test_gemm_dma_tiles_equal_the_other_forms(be, m, ns, k):
+    """Every tile of the DMA form (256 CUs), alone and in a list, partial in
+    both directions and for one stage of k up: the same products in a list with
+    one of k = 96, which the DMA form does not take, run on the forms without it
+    and agree bit for bit (one MFMA chain per element)."""
+    rsv = _rsv()
+    rng = np.random.default_rng(m + k)
+    f16 = lambda *shape: be.tensor(rng.standard_normal(shape).astype(np.float32), dtype=rsv.F16)  # noqa: E731
+    x, ws = f16(m, k), [f16(n, k) for n in ns]
+    outs = [[be.tensor(n=m * n) for n in ns] for _ in range(2)]
+    lists = [[rsv.MmJob(w, None, n, k, x, y, NONE, 0, NONE, NONE, NONE, 0) for w, n, y in zip(ws, ns, ys)] for ys in outs]
+    lists[1].append(rsv.MmJob(f16(64, 96), None, 64, 96, f16(m, 96), be.tensor(n=m * 64), NONE, 0, NONE, NONE, NONE, 0))
+    if len(ns) == 1:
+        be.call("rsv_gemm_ex", x, ws[0], None, outs[0][0], m, ns[0], k, 0, NONE, NONE, NONE)
+        lists = lists[1:]
+    for jobs in lists:
+        be.call("rsv_gemm_multi", ctypes.cast((rsv.MmJob * len(jobs))(*jobs), ctypes.c_void_p), len(jobs), m)
+    for a, b, n in zip(*outs, ns):
+        assert np.array_equal(be.get(a, m * n).view(np.uint32), be.get(b, m * n).view(np.uint32)), n
 
 
 @pytest.mark.parametrize("m", [1030, 4096])

@@ -476,7 +476,7 @@ __global__ __launch_bounds__(256, BKT == 64 ? 3 : 2) void k_gemm3_multi(GemmJobs
 //     a later 16 k in flight during them.
 //   - What bounds it: the large tiles, with the chip full, the matrix pipes at
 //     the clock the power leaves (256x160 at 4096 x 10240 x 2560: 1020
-//     TFLOP/s); the small ones a CU's copy rate from L2 to LDS (about 80 GB/s
+//     TFLOP/s); the small ones a CU's copy rate from L2 to LDS (about 65 GB/s
 //     a CU: 0.5 us a stage of 32 KB while its MFMAs take 0.25), so what does
 //     not fill the chip wants more and smaller tiles, down to 64x64.
 //   - The MFMA is the one of k_gemm2/3 (v_mfma_f32_32x32x16_f16, lane l

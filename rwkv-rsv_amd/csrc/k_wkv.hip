@@ -1134,11 +1134,12 @@ __global__ __launch_bounds__(256 / RPL) void k_wkv7_seq_rows(
 //     (q, e) is S[row = l%16][column = 16q + 4(l/16) + e].  As the B operand of
 //     k-step (q, e) it is used in place: the four k of a step may be any four
 //     columns, and A's lane reads the same ones, one 16-byte LDS read per q.
-//     U's result layout (token 4(l/16) + e, row l%16) is B-operand layout too.
+//     U's result layout (token 4e + l/16, see mm_row; row l%16) is B-operand layout too.
 //   - LDS: rows of 68 floats, read as 16 rows x one 16-byte piece, as 4 rows x 16
 //     consecutive floats and as whole rows; rt has rows of 64 with piece p of
 //     row t at p ^ t (160 KB hold eight chunks), rows of 16 keep piece p at
-//     p ^ (t/4).  All reads are free of bank conflicts.
+//     p ^ (t/4), so that those reads meet no bank twice (conflicts counted over all
+//     accesses, stores too: 13 to 16 % of the LDS's active cycles).
 //   - A chunk whose Gram products pass 2^40 or are not finite (strong decays, or
 //     inputs not finite), where 0 * inf would reach the chunk's earlier tokens, is
 //     stepped token by token, from memory, by the waves that hold the state, and so
@@ -1419,8 +1420,7 @@ __device__ __forceinline__ void mm_consume(const WkvChunk &c, const WkvChunk &n,
                                            f4_t &y, int lane) {
     const int l16 = lane & 15, g = lane >> 4;
     // The reads of a later phase go out one after each product of the phase
-    // before it (the groups below order them): fp32 products leave a wave's issue
-    // slots to LDS reads, but not to its VALU.
+    // before it (the groups below order them).
     float kh[4][4], bh[4][4];
 #pragma unroll
     for (int e = 0; e < 4; e++)
@@ -1566,8 +1566,9 @@ __device__ __forceinline__ int nth_long(const uint32_t *__restrict__ seg_len, in
 // rows, 16 each, through the NP chunks of the other.
 //   <4, 4>: the preparing is done once per head; 8 waves, one block per CU.
 //   <1, 3>: a quarter of the rows per block, for launches that leave CUs idle.
-//     fp32 MFMA holds its SIMD's VALU for half of its 32 cycles, so a preparing
-//     wave beside a passing one slows both; here each has a SIMD of its own.
+//     Here a preparing and a passing wave have a SIMD each, and neither waits for
+//     the other's products (32 cycles each): 1 x 512 at 40 heads 71 us, whole
+//     heads 83.
 // (Bounds of 512 threads for both: with one wave per SIMD allowed for <1, 3> the
 // compiler keeps the sums in AGPRs and moves them through VGPRs for each addition.)
 template <int NC, int NP>
